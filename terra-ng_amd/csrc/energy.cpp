@@ -33,6 +33,7 @@ struct tng_energy_s {
     std::vector<std::unique_ptr<tng_vector>> pool;
     tng_vector *g = nullptr, *tmp = nullptr, *q = nullptr, *diag = nullptr, *ones = nullptr, *t_backup = nullptr;
     std::vector<tng_vector *> fg;  // FGMRES work space: 2m + 4 scalars
+    tng::DevBuf tau, bdiag;        // SUPG tau per wedge and boundary diagonal of the step's velocity
     double h = 0.0;
 };
 
@@ -209,6 +210,25 @@ void energy_step(tng_energy_s &e, double dt, tng_solve_report &rep)
     e.A->supg_dt = dt;
     e.A_neumann->supg_dt = dt;
     e.A_neumann_diag->supg_dt = dt;
+    // the velocity does not change within a step: tau and the boundary rows'
+    // diagonal once for all its applies
+    const tng_domain &m = *e.temp->mesh;
+    if (!e.tau.p) e.tau.alloc(supg_tau_count(m) * sizeof(double));
+    if (!e.bdiag.p) e.bdiag.alloc(2 * (size_t)m.nlat * sizeof(double));
+    struct StepData {
+        tng_operator *ops[3];
+        StepData(tng_energy_s &e) : ops{e.A.get(), e.A_neumann.get(), e.A_neumann_diag.get()}
+        {
+            for (tng_operator *op : ops) op->supg_step_tau = e.tau.as<double>();
+            ops[0]->supg_step_bdiag = e.bdiag.as<double>();
+        }
+        ~StepData()
+        {
+            for (tng_operator *op : ops) op->supg_step_tau = op->supg_step_bdiag = nullptr;
+        }
+    } step_data(e);
+    supg_tau(*e.A, e.tau.as<double>(), s);
+    supg_boundary_diagonal(*e.A, e.tau.as<double>(), e.bdiag.as<double>(), s);
     // inverse diagonal at the step's dt
     op_apply(*e.A_neumann_diag, *e.ones, *e.diag);
     launch_invert(*e.diag, s);

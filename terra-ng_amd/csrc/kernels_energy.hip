@@ -12,8 +12,19 @@
 // velocity and tau the quadrature-weighted mean of supg_tau over the points
 // (h = r_2 - r_1).  Boundary-layer rows keep their diagonal entry only; the
 // diagonal mode keeps every row's diagonal entry; the lumped mass takes the
-// row sums m sum_q w_q |det J_q| phi_i.  One thread per cell writes the 12
-// wedge-node partials of the cell; a per-node gather sums them (no atomics).
+// row sums m sum_q w_q |det J_q| phi_i.
+//
+// Formulation used here.  The Jacobian at lateral point s and radius r is
+// [e1, e2, p_s] diag(r, r, h/2) with e1, e2 the triangle's edges and p_s the
+// point on it, so its inverse transpose has the columns M0_s / r, M1_s / r,
+// M2 / (h/2) and |det J| = |det L| r^2 h/2, where M0_s = (e2 x p_s) / det L,
+// M1_s = (p_s x e1) / det L, M2 = (e1 x e2) / det L are lateral data alone.
+// With the contravariant velocity (u.M0_s / r, u.M1_s / r, u.M2 / (h/2)) and
+// the Gram products M_i.M_j the bilinear form needs no physical gradients:
+// the reference-space derivatives of T and of the test functions (three
+// numbers per point each) carry everything.  tau depends on the velocity
+// only; it comes from a kernel of its own (six square roots, hyperbolic
+// tangents and divisions per wedge), once per energy step.
 #include <algorithm>
 
 #include "tng_internal.hpp"
@@ -37,130 +48,465 @@ __device__ double supg_tau_dev(double vel_norm, double kappa, double h, double p
     return tau > tau_max ? tau_max : tau;
 }
 
+// Felippa rule: lateral point s has weight 2/3 at corner kPoint[s] and 1/6 at
+// the two others, two radial Gauss points, all weights 1/6.
+constexpr double kGauss = 0.5773502691896257;
+
 struct SupgArgs {
     const double *src, *u0, *u1, *u2;
     const double *coords, *radii;
-    const uint8_t *bmask;
-    double *partial;  // (cell, wedge, 6)
+    const uint8_t *sd_cmb, *sd_surf;
+    const double *tau;    // (cell, wedge), nullptr: no streamline term
+    const double *bdiag;  // (lateral node, side): diagonal entries of the treated boundary rows
+    double *partial;      // (lateral cell, corner, level)
+    double *dst;
     double kappa, dt, mass;
-    int treat_boundary, diagonal, lumped, supg;
+    int treat_boundary, lumped, add;
     int nsd, nx, nr;
+    int lr, lc;     // log2 of the radial and lateral cells per subdomain
+    int plen, lseg; // entries per (lateral cell, corner), log2 of the cells per radial segment
+    int64_t ncell;
 };
 
-__global__ __launch_bounds__(128) void supg_cell_kernel(const SupgArgs a)
+// Lateral data of one triangle at the three lateral points.
+struct SupgGeom {
+    double m0[3][3], m1[3][3], g00[3], g01[3], g11[3], g02[3], g12[3];
+    double m2[3], g22, det;
+};
+
+// Fills entry (w, s) of the geometry of lateral cell col.
+__device__ __forceinline__ void supg_geometry(const SupgArgs &a, int64_t col, int w, int s, SupgGeom &G)
 {
-    const int nx = a.nx, nr = a.nr, nc = nx - 1, ncr = nr - 1;
-    const int64_t ncell = (int64_t)a.nsd * nc * nc * ncr;
-    const int64_t cell = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (cell >= ncell) return;
-    const int rc = (int)(cell % ncr);
-    int64_t t = cell / ncr;
-    const int yc = (int)(t % nc);
-    t /= nc;
-    const int xc = (int)(t % nc);
-    const int sd = (int)(t / nc);
-    const double r1 = a.radii[(int64_t)sd * nr + rc], r2 = a.radii[(int64_t)sd * nr + rc + 1];
-    const double h = r2 - r1;
-    const uint8_t cmb = 2 | 4, surf = 2 | 8;
-    const bool at_cmb = (a.bmask[(((int64_t)sd * nx + xc) * nx + yc) * nr + rc] & cmb) == cmb;
-    const bool at_surf = (a.bmask[(((int64_t)sd * nx + xc) * nx + yc) * nr + rc + 1] & surf) == surf;
-    const double qx[3] = {0.6666666666666666, 0.1666666666666667, 0.1666666666666667};
-    const double qy[3] = {0.1666666666666667, 0.6666666666666666, 0.1666666666666667};
-    const double qz[2] = {-0.5773502691896257, 0.5773502691896257};
-    const double qw = 0.1666666666666667;
-    for (int w = 0; w < 2; ++w) {
-        double P[3][3], Tn[6], U[6][3];
-        bool bnd[6];
-        for (int n = 0; n < 6; ++n) {
-            const int64_t lcol = ((int64_t)sd * nx + xc + kEW[w][n][0]) * nx + yc + kEW[w][n][1];
-            const int64_t i = lcol * nr + rc + kEW[w][n][2];
-            if (n < 3)
-                for (int d = 0; d < 3; ++d) P[n][d] = a.coords[3 * lcol + d];
-            Tn[n] = a.src[i];
-            U[n][0] = a.u0[i];
-            U[n][1] = a.u1[i];
-            U[n][2] = a.u2[i];
-            bnd[n] = a.treat_boundary && ((at_cmb && n < 3) || (at_surf && n >= 3));
-        }
-        // velocity at the points and tau
-        double uq[6][3];
-        double tau_acc = 0.0, wacc = 0.0;
-        for (int q = 0; q < 6; ++q) {
-            const double xi = qx[q % 3], eta = qy[q % 3], zeta = qz[q / 3];
-            const double Nl[3] = {1.0 - xi - eta, xi, eta}, Nr[2] = {0.5 * (1.0 - zeta), 0.5 * (1.0 + zeta)};
+    const int nc = a.nx - 1;
+    const int yc = (int)(col & (nc - 1)), xc = (int)((col >> a.lc) & (nc - 1)), sd = (int)(col >> (2 * a.lc));
+    double P[3][3];
+    for (int n = 0; n < 3; ++n) {
+        const double *c = a.coords + 3 * (((int64_t)sd * a.nx + xc + kEW[w][n][0]) * a.nx + yc + kEW[w][n][1]);
+        for (int d = 0; d < 3; ++d) P[n][d] = c[d];
+    }
+    const int ks = s == 0 ? 1 : (s == 1 ? 2 : 0);
+    double e1[3], e2[3], p[3];
+    for (int d = 0; d < 3; ++d) {
+        e1[d] = P[1][d] - P[0][d];
+        e2[d] = P[2][d] - P[0][d];
+        const double pk = ks == 0 ? P[0][d] : (ks == 1 ? P[1][d] : P[2][d]);
+        p[d] = (P[0][d] + P[1][d] + P[2][d]) * (1.0 / 6.0) + 0.5 * pk;
+    }
+    auto cross = [](const double *x, const double *y, double *o) {
+        o[0] = x[1] * y[2] - x[2] * y[1];
+        o[1] = x[2] * y[0] - x[0] * y[2];
+        o[2] = x[0] * y[1] - x[1] * y[0];
+    };
+    auto dot = [](const double *x, const double *y) { return x[0] * y[0] + x[1] * y[1] + x[2] * y[2]; };
+    double n[3], m0[3], m1[3];
+    cross(e1, e2, n);
+    cross(e2, p, m0);
+    cross(p, e1, m1);
+    const double det = dot(n, p), id = 1.0 / det;
+    for (int d = 0; d < 3; ++d) {
+        n[d] *= id;
+        m0[d] *= id;
+        m1[d] *= id;
+        G.m0[s][d] = m0[d];
+        G.m1[s][d] = m1[d];
+        if (s == 0) G.m2[d] = n[d];
+    }
+    G.g00[s] = dot(m0, m0);
+    G.g01[s] = dot(m0, m1);
+    G.g11[s] = dot(m1, m1);
+    G.g02[s] = dot(m0, n);
+    G.g12[s] = dot(m1, n);
+    if (s == 0) {
+        G.g22 = dot(n, n);
+        G.det = fabs(det);
+    }
+}
+
+// Diagonal entries of the six rows of one wedge, without the lumped mass.
+__device__ __forceinline__ void supg_wedge_diag(const SupgArgs &a, const SupgGeom *geom, int gi, const double (&ub)[3][4],
+                                                const double (&ut)[3][4], double r1, double r2, double tau,
+                                                double (&db)[3], double (&dt_)[3])
+{
+    const double gr = 0.5 * (r2 - r1), igr = 1.0 / gr;
+    const double mass = a.lumped ? 0.0 : a.mass;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) db[k] = dt_[k] = 0.0;
+#pragma unroll 1
+    for (int z = 0; z < 2; ++z) {
+        const double zeta = z == 0 ? -kGauss : kGauss;
+        const double n0 = 0.5 * (1.0 - zeta), n1 = 0.5 * (1.0 + zeta);
+        // the lateral data is read again for each z (an opaque index): kept
+        // over the loop it costs 76 registers and with them the occupancy
+        asm volatile("" : "+v"(gi));
+        const SupgGeom &G = geom[gi];
+        const double r = r1 + gr * (1.0 + zeta), ir = 1.0 / r, wz = G.det * r * r * gr * (1.0 / 6.0);
+#pragma unroll
+        for (int s = 0; s < 3; ++s) {
+            const int ks = s == 0 ? 1 : (s == 1 ? 2 : 0);
+            double u[3];
+#pragma unroll
             for (int d = 0; d < 3; ++d) {
-                double s = 0.0;
-                for (int n = 0; n < 6; ++n) s += U[n][d] * (Nl[n % 3] * Nr[n / 3]);
-                uq[q][d] = s;
+                const double z0 = n0 * ub[d][0] + n1 * ut[d][0], z1 = n0 * ub[d][1] + n1 * ut[d][1],
+                             z2 = n0 * ub[d][2] + n1 * ut[d][2];
+                u[d] = (z0 + z1 + z2) * (1.0 / 6.0) + 0.5 * (ks == 0 ? z0 : (ks == 1 ? z1 : z2));
             }
-            const double vn = sqrt(uq[q][0] * uq[q][0] + uq[q][1] * uq[q][1] + uq[q][2] * uq[q][2]);
-            tau_acc += supg_tau_dev(vn, a.kappa, h, 1e-08) * qw;
-            wacc += qw;
-        }
-        const double tau = a.supg ? (wacc > 0.0 ? tau_acc / wacc : 0.0) : 0.0;
-        double out[6] = {0, 0, 0, 0, 0, 0}, diag[6] = {0, 0, 0, 0, 0, 0}, lmass[6] = {0, 0, 0, 0, 0, 0};
-        for (int q = 0; q < 6; ++q) {
-            const double xi = qx[q % 3], eta = qy[q % 3], zeta = qz[q / 3];
-            const double Nl[3] = {1.0 - xi - eta, xi, eta}, Nr[2] = {0.5 * (1.0 - zeta), 0.5 * (1.0 + zeta)};
-            const double r = r1 + 0.5 * (r2 - r1) * (1.0 + zeta), gr = 0.5 * (r2 - r1);
-            double J[3][3];
-            for (int d = 0; d < 3; ++d) {
-                J[d][0] = (P[1][d] - P[0][d]) * r;
-                J[d][1] = (P[2][d] - P[0][d]) * r;
-                J[d][2] = (Nl[0] * P[0][d] + Nl[1] * P[1][d] + Nl[2] * P[2][d]) * gr;
+            const double al = (u[0] * G.m0[s][0] + u[1] * G.m0[s][1] + u[2] * G.m0[s][2]) * ir;
+            const double be = (u[0] * G.m1[s][0] + u[1] * G.m1[s][1] + u[2] * G.m1[s][2]) * ir;
+            const double ga = (u[0] * G.m2[0] + u[1] * G.m2[1] + u[2] * G.m2[2]) * igr;
+            const double h00 = G.g00[s] * ir * ir, h01 = G.g01[s] * ir * ir, h11 = G.g11[s] * ir * ir,
+                         h02 = G.g02[s] * ir * igr, h12 = G.g12[s] * ir * igr, h22 = G.g22 * igr * igr;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const double nl = k == ks ? 2.0 / 3.0 : 1.0 / 6.0;
+                const double lx = k == 0 ? -1.0 : (k == 1 ? 1.0 : 0.0), ly = k == 0 ? -1.0 : (k == 2 ? 1.0 : 0.0);
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    const double nr = t == 0 ? n0 : n1, dr = t == 0 ? -0.5 : 0.5;
+                    const double fx = lx * nr, fy = ly * nr, fz = nl * dr, phi = nl * nr;
+                    const double ug = fx * al + fy * be + fz * ga;
+                    const double gg = fx * fx * h00 + fy * fy * h11 + fz * fz * h22 +
+                                      2.0 * (fx * fy * h01 + fx * fz * h02 + fy * fz * h12);
+                    const double v = wz * (mass * phi * phi + a.dt * (a.kappa * gg + ug * phi + tau * ug * ug));
+                    if (t == 0) db[k] += v;
+                    else dt_[k] += v;
+                }
             }
-            const double c00 = J[1][1] * J[2][2] - J[1][2] * J[2][1], c01 = J[1][2] * J[2][0] - J[1][0] * J[2][2],
-                         c02 = J[1][0] * J[2][1] - J[1][1] * J[2][0];
-            const double det = J[0][0] * c00 + J[0][1] * c01 + J[0][2] * c02;
-            const double id = 1.0 / det;
-            // (J^{-T})_{ab}
-            double iT[3][3];
-            iT[0][0] = c00 * id; iT[0][1] = c01 * id; iT[0][2] = c02 * id;
-            iT[1][0] = (J[0][2] * J[2][1] - J[0][1] * J[2][2]) * id;
-            iT[1][1] = (J[0][0] * J[2][2] - J[0][2] * J[2][0]) * id;
-            iT[1][2] = (J[0][1] * J[2][0] - J[0][0] * J[2][1]) * id;
-            iT[2][0] = (J[0][1] * J[1][2] - J[0][2] * J[1][1]) * id;
-            iT[2][1] = (J[0][2] * J[1][0] - J[0][0] * J[1][2]) * id;
-            iT[2][2] = (J[0][0] * J[1][1] - J[0][1] * J[1][0]) * id;
-            const double wd = qw * fabs(det);
-            const double gxi[3] = {-1.0, 1.0, 0.0}, geta[3] = {-1.0, 0.0, 1.0}, grad_rad[2] = {-0.5, 0.5};
-            double g[6][3], phi[6];
-            for (int n = 0; n < 6; ++n) {
-                const double gref[3] = {gxi[n % 3] * Nr[n / 3], geta[n % 3] * Nr[n / 3], Nl[n % 3] * grad_rad[n / 3]};
-                for (int b = 0; b < 3; ++b) g[n][b] = iT[b][0] * gref[0] + iT[b][1] * gref[1] + iT[b][2] * gref[2];
-                phi[n] = Nl[n % 3] * Nr[n / 3];
-            }
-            // trial values with the Dirichlet columns removed
-            double Th = 0.0, gT[3] = {0.0, 0.0, 0.0};
-            for (int n = 0; n < 6; ++n) {
-                const double tv = bnd[n] ? 0.0 : Tn[n];
-                Th += phi[n] * tv;
-                for (int b = 0; b < 3; ++b) gT[b] += g[n][b] * tv;
-            }
-            const double ugT = uq[q][0] * gT[0] + uq[q][1] * gT[1] + uq[q][2] * gT[2];
-            const double As = a.mass * Th + a.dt * ugT;
-            const double As_nomass = a.dt * ugT;
-            double Bv[3];
-            for (int b = 0; b < 3; ++b) Bv[b] = a.dt * a.kappa * gT[b] + a.dt * tau * ugT * uq[q][b];
-            for (int i = 0; i < 6; ++i) {
-                const double gB = g[i][0] * Bv[0] + g[i][1] * Bv[1] + g[i][2] * Bv[2];
-                out[i] += wd * (phi[i] * (a.lumped ? As_nomass : As) + gB);
-                // diagonal entry (M_ii + A_ii)
-                const double ugi = uq[q][0] * g[i][0] + uq[q][1] * g[i][1] + uq[q][2] * g[i][2];
-                const double gg = g[i][0] * g[i][0] + g[i][1] * g[i][1] + g[i][2] * g[i][2];
-                const double mii = a.mass * phi[i] * phi[i];
-                diag[i] += wd * ((a.lumped ? 0.0 : mii) + a.dt * (a.kappa * gg + ugi * phi[i] + tau * ugi * ugi));
-                lmass[i] += wd * a.mass * phi[i];
-            }
-        }
-        double *o = a.partial + (cell * 2 + w) * 6;
-        for (int i = 0; i < 6; ++i) {
-            double v;
-            if (a.diagonal || bnd[i]) v = (diag[i] + (a.lumped ? lmass[i] : 0.0)) * Tn[i];
-            else v = out[i] + (a.lumped ? lmass[i] * Tn[i] : 0.0);
-            o[i] = v;
         }
     }
+}
+
+// The wedge's action on the nodal values of its three corners, bottom (tb,
+// ob) and top (tt, ot); zero_b / zero_t: the Dirichlet columns left out.
+__device__ __forceinline__ void supg_wedge_apply(const SupgArgs &a, const SupgGeom *geom, int gi, const double (&Tb)[4],
+                                                 const double (&Tt)[4], bool zero_b, bool zero_t,
+                                                 const double (&ub)[3][4], const double (&ut)[3][4], double r1,
+                                                 double r2, double tau, double (&ob)[3], double (&ot)[3])
+{
+    double tb[3], tt[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        tb[k] = zero_b ? 0.0 : Tb[k];
+        tt[k] = zero_t ? 0.0 : Tt[k];
+    }
+    const double gr = 0.5 * (r2 - r1), igr = 1.0 / gr;
+    const double mass = a.lumped ? 0.0 : a.mass, dk = a.dt * a.kappa, dtau = a.dt * tau;
+    const double D[3] = {0.5 * (tt[0] - tb[0]), 0.5 * (tt[1] - tb[1]), 0.5 * (tt[2] - tb[2])};
+    const double D6 = (D[0] + D[1] + D[2]) * (1.0 / 6.0);
+#pragma unroll 1
+    for (int z = 0; z < 2; ++z) {
+        const double zeta = z == 0 ? -kGauss : kGauss;
+        const double n0 = 0.5 * (1.0 - zeta), n1 = 0.5 * (1.0 + zeta);
+        // the lateral data is read again for each z (an opaque index): kept
+        // over the loop it costs 76 registers and with them the occupancy
+        asm volatile("" : "+v"(gi));
+        const SupgGeom &G = geom[gi];
+        const double r = r1 + gr * (1.0 + zeta), ir = 1.0 / r, wz = G.det * r * r * gr * (1.0 / 6.0);
+        double T[3], u[3][3], U6[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            T[k] = n0 * tb[k] + n1 * tt[k];
+#pragma unroll
+            for (int d = 0; d < 3; ++d) u[k][d] = n0 * ub[d][k] + n1 * ut[d][k];
+        }
+#pragma unroll
+        for (int d = 0; d < 3; ++d) U6[d] = (u[0][d] + u[1][d] + u[2][d]) * (1.0 / 6.0);
+        const double T6 = (T[0] + T[1] + T[2]) * (1.0 / 6.0);
+        const double ax = T[1] - T[0], ay = T[2] - T[0];
+        double L[3] = {0.0, 0.0, 0.0}, R[3] = {0.0, 0.0, 0.0}, S6 = 0.0, Z6 = 0.0, Fx = 0.0, Fy = 0.0;
+#pragma unroll
+        for (int s = 0; s < 3; ++s) {
+            const int ks = s == 0 ? 1 : (s == 1 ? 2 : 0);
+            const double q[3] = {U6[0] + 0.5 * u[ks][0], U6[1] + 0.5 * u[ks][1], U6[2] + 0.5 * u[ks][2]};
+            const double al = (q[0] * G.m0[s][0] + q[1] * G.m0[s][1] + q[2] * G.m0[s][2]) * ir;
+            const double be = (q[0] * G.m1[s][0] + q[1] * G.m1[s][1] + q[2] * G.m1[s][2]) * ir;
+            const double ga = (q[0] * G.m2[0] + q[1] * G.m2[1] + q[2] * G.m2[2]) * igr;
+            const double c = D6 + 0.5 * D[ks];
+            const double ugT = al * ax + be * ay + ga * c;
+            const double S = wz * (mass * (T6 + 0.5 * T[ks]) + a.dt * ugT);
+            // diffusive flux in the dual basis: scaled derivatives, then the Gram products
+            const double px = ax * ir, py = ay * ir, pz = c * igr, st = dtau * ugT;
+            const double fx = wz * (dk * ir * (G.g00[s] * px + G.g01[s] * py + G.g02[s] * pz) + st * al);
+            const double fy = wz * (dk * ir * (G.g01[s] * px + G.g11[s] * py + G.g12[s] * pz) + st * be);
+            const double fz = wz * (dk * igr * (G.g02[s] * px + G.g12[s] * py + G.g22 * pz) + st * ga);
+            Fx += fx;
+            Fy += fy;
+            S6 += S;
+            Z6 += fz;
+            L[ks] += 0.5 * S;
+            R[ks] += 0.5 * fz;
+        }
+        S6 *= 1.0 / 6.0;
+        Z6 *= 1.0 / 6.0;
+        L[0] += S6 - (Fx + Fy);
+        L[1] += S6 + Fx;
+        L[2] += S6 + Fy;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const double rk = 0.5 * (Z6 + R[k]);
+            ob[k] += n0 * L[k] - rk;
+            ot[k] += n1 * L[k] + rk;
+        }
+    }
+}
+
+// Row sums of the wedge's mass (lumped mode): the same for the three corners.
+__device__ __forceinline__ void supg_lumped_mass(const SupgArgs &a, const SupgGeom &G, double r1, double r2,
+                                                 double &mb, double &mt)
+{
+    const double gr = 0.5 * (r2 - r1);
+    mb = mt = 0.0;
+    for (int z = 0; z < 2; ++z) {
+        const double zeta = z == 0 ? -kGauss : kGauss;
+        const double r = r1 + gr * (1.0 + zeta), wz = a.mass * G.det * r * r * gr * (1.0 / 6.0);
+        mb += 0.5 * (1.0 - zeta) * wz;
+        mt += 0.5 * (1.0 + zeta) * wz;
+    }
+}
+
+struct SupgCell {
+    int64_t col;  // lateral cell
+    int rc, xc, yc, sd;
+};
+
+__device__ __forceinline__ SupgCell supg_cell_of(const SupgArgs &a, int64_t cell)
+{
+    const int nc = a.nx - 1;
+    SupgCell c;
+    c.rc = (int)(cell & ((1 << a.lr) - 1));
+    c.col = cell >> a.lr;
+    c.yc = (int)(c.col & (nc - 1));
+    c.xc = (int)((c.col >> a.lc) & (nc - 1));
+    c.sd = (int)(c.col >> (2 * a.lc));
+    return c;
+}
+
+// One thread per cell (lanes along r), its two wedges together: the eight
+// nodes are loaded once, the lateral data of the block's columns is formed
+// once per block in LDS.  A corner column's contributions to a node level (the
+// cell above as its bottom, the cell below as its top) are summed through LDS,
+// so a lateral cell writes four values per level instead of twelve per cell
+// (84 MB against 250 MB at level 6), and the gather below reads four.  Bound
+// by FP64 arithmetic at two waves per SIMD (221 VGPRs).  Level 6 (2.6 M
+// cells): 167 us + 24 us for the gather, against 721 us + 140 us with the
+// Jacobian inverse, tau and every row's diagonal formed at each of the six
+// points of each wedge and twelve partials per cell; tau takes 257 us, once
+// per step.
+template <bool DIAG> __global__ __launch_bounds__(256) void supg_cell_kernel(const SupgArgs a)
+{
+    extern __shared__ double smem[];
+    const int tb_ = blockDim.x, ncr = 1 << a.lr;
+    SupgGeom *geom = reinterpret_cast<SupgGeom *>(smem);
+    const int64_t cell0 = (int64_t)blockIdx.x * tb_, ncol = a.ncell >> a.lr;
+    const int64_t col0 = cell0 >> a.lr;
+    const int cols = tb_ > ncr ? tb_ >> a.lr : 1;
+    double *tops = smem + cols * 2 * (sizeof(SupgGeom) / sizeof(double));  // (corner, thread)
+    for (int t = threadIdx.x; t < cols * 6; t += tb_) {
+        const int64_t col = min(col0 + t / 6, ncol - 1);
+        supg_geometry(a, col, (t / 3) & 1, t % 3, geom[t / 3]);
+    }
+    __syncthreads();
+    const int64_t cell = min(cell0 + (int64_t)threadIdx.x, a.ncell - 1);
+    const bool live = cell0 + threadIdx.x < a.ncell;
+    const SupgCell c = supg_cell_of(a, cell);
+    const int nx = a.nx, nr = a.nr;
+    const double r1 = a.radii[(int64_t)c.sd * nr + c.rc], r2 = a.radii[(int64_t)c.sd * nr + c.rc + 1];
+    const bool zero_b = a.treat_boundary && c.rc == 0 && a.sd_cmb[c.sd];
+    const bool zero_t = a.treat_boundary && c.rc == ncr - 1 && a.sd_surf[c.sd];
+    // corners 00, 10, 01, 11
+    double Tb[4], Tt[4], Ub[3][4], Ut[3][4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int64_t i = (((int64_t)c.sd * nx + c.xc + (k & 1)) * nx + c.yc + (k >> 1)) * nr + c.rc;
+        Tb[k] = a.src[i];
+        Tt[k] = a.src[i + 1];
+        Ub[0][k] = a.u0[i];
+        Ut[0][k] = a.u0[i + 1];
+        Ub[1][k] = a.u1[i];
+        Ut[1][k] = a.u1[i + 1];
+        Ub[2][k] = a.u2[i];
+        Ut[2][k] = a.u2[i + 1];
+    }
+    double ob[4] = {0, 0, 0, 0}, ot[4] = {0, 0, 0, 0};
+    // A real loop over the two wedges: the corners of the second, (3, 2, 1),
+    // are those of the first after the four are turned end for end, so one
+    // body serves both and its registers are live once (unrolled, the compiler
+    // keeps both wedges' lateral data and interpolants: 294 VGPRs, one wave
+    // per SIMD).
+#pragma unroll 1
+    for (int w = 0; w < 2; ++w) {
+        const SupgGeom &G = geom[2 * (c.col - col0) + w];
+        const double tw = a.tau ? a.tau[2 * cell + w] : 0.0;
+        double wb[3] = {0, 0, 0}, wt[3] = {0, 0, 0}, mb = 0.0, mt = 0.0;
+        if constexpr (DIAG)
+            supg_wedge_diag(a, geom, 2 * (int)(c.col - col0) + w, Ub, Ut, r1, r2, tw, wb, wt);
+        else
+            supg_wedge_apply(a, geom, 2 * (int)(c.col - col0) + w, Tb, Tt, zero_b, zero_t, Ub, Ut, r1, r2, tw, wb, wt);
+        if (a.lumped) supg_lumped_mass(a, G, r1, r2, mb, mt);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            if constexpr (DIAG) {
+                ob[k] += (wb[k] + mb) * Tb[k];
+                ot[k] += (wt[k] + mt) * Tt[k];
+            } else {
+                ob[k] += wb[k] + mb * Tb[k];
+                ot[k] += wt[k] + mt * Tt[k];
+            }
+        }
+        auto turn = [](auto &v) {
+            for (int k = 0; k < 2; ++k) {
+                const double t = v[k];
+                v[k] = v[3 - k];
+                v[3 - k] = t;
+            }
+        };
+        turn(Tb);
+        turn(Tt);
+        turn(ob);
+        turn(ot);
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            turn(Ub[d]);
+            turn(Ut[d]);
+        }
+    }
+    // level rc of a corner column: this cell's bottom and the top of the cell
+    // below; a segment's first cell has no cell below, its last one also
+    // writes the level above
+    const int seg = (1 << a.lseg) - 1;
+    const bool first = (c.rc & seg) == 0, last = (c.rc & seg) == seg || c.rc == ncr - 1;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) tops[k * tb_ + threadIdx.x] = ot[k];
+    __syncthreads();
+    if (!live) return;
+    double *o = a.partial + c.col * 4 * a.plen + c.rc + (c.rc >> a.lseg);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        o[(int64_t)k * a.plen] = first ? ob[k] : ob[k] + tops[k * tb_ + threadIdx.x - 1];
+        if (last) o[(int64_t)k * a.plen + 1] = ot[k];
+    }
+}
+
+// Node values from the four lateral cells around a node; treated boundary
+// rows are their diagonal entry times the value.
+__global__ __launch_bounds__(256) void supg_gather_kernel(const SupgArgs a, const Index4 idx)
+{
+    const uint32_t n = (uint32_t)a.nsd * a.nx * a.nx * a.nr;
+    const uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
+    if (gid >= n) return;
+    int sd, X, Y, l;
+    idx.decode(gid, sd, X, Y, l);
+    const int nc = a.nx - 1, ncr = a.nr - 1;
+    const int seg = min(l, ncr - 1) >> a.lseg;
+    const bool seam = l < ncr && l > 0 && (l & ((1 << a.lseg) - 1)) == 0;
+    double v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int xc = X - (k & 1), yc = Y - (k >> 1);
+        v[k] = 0.0;
+        if (xc >= 0 && xc < nc && yc >= 0 && yc < nc) {
+            const double *p = a.partial + ((((int64_t)sd * nc + xc) * nc + yc) * 4 + k) * a.plen + l + seg;
+            v[k] = p[0];
+            if (seam) v[k] += p[-1];
+        }
+    }
+    double s = (v[0] + v[1]) + (v[2] + v[3]);
+    if (a.bdiag) {
+        const uint32_t lcol = ((uint32_t)sd * a.nx + X) * a.nx + Y;
+        if (l == 0 && a.sd_cmb[sd]) s = a.bdiag[2 * lcol] * a.src[gid];
+        else if (l == ncr && a.sd_surf[sd]) s = a.bdiag[2 * lcol + 1] * a.src[gid];
+    }
+    a.dst[gid] = a.add ? a.dst[gid] + s : s;
+}
+
+// tau per wedge: one thread per cell, the velocity at the six points.
+__global__ __launch_bounds__(256) void supg_tau_kernel(const SupgArgs a, double *tau)
+{
+    const int64_t cell = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (cell >= a.ncell) return;
+    const SupgCell c = supg_cell_of(a, cell);
+    const int nx = a.nx, nr = a.nr;
+    const double h = a.radii[(int64_t)c.sd * nr + c.rc + 1] - a.radii[(int64_t)c.sd * nr + c.rc];
+    double U[2][4][3];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int64_t i = (((int64_t)c.sd * nx + c.xc + (k & 1)) * nx + c.yc + (k >> 1)) * nr + c.rc;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            U[t][k][0] = a.u0[i + t];
+            U[t][k][1] = a.u1[i + t];
+            U[t][k][2] = a.u2[i + t];
+        }
+    }
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+        constexpr int kC[2][3] = {{0, 1, 2}, {3, 2, 1}};
+        double acc = 0.0;
+#pragma unroll
+        for (int z = 0; z < 2; ++z) {
+            const double n0 = z == 0 ? 0.5 * (1.0 + kGauss) : 0.5 * (1.0 - kGauss), n1 = 1.0 - n0;
+#pragma unroll
+            for (int s = 0; s < 3; ++s) {
+                const int ks = s == 0 ? 1 : (s == 1 ? 2 : 0);
+                double vn = 0.0;
+#pragma unroll
+                for (int d = 0; d < 3; ++d) {
+                    double u = 0.0;
+#pragma unroll
+                    for (int k = 0; k < 3; ++k)
+                        u += (k == ks ? 2.0 / 3.0 : 1.0 / 6.0) * (n0 * U[0][kC[w][k]][d] + n1 * U[1][kC[w][k]][d]);
+                    vn += u * u;
+                }
+                acc += supg_tau_dev(sqrt(vn), a.kappa, h, 1e-08);
+            }
+        }
+        tau[2 * cell + w] = acc * (1.0 / 6.0);
+    }
+}
+
+// Diagonal entries of the treated boundary rows, per lateral node copy and
+// side: one thread per entry, gathering over the wedges around it.
+__global__ __launch_bounds__(64) void supg_bdiag_kernel(const SupgArgs a, double *bdiag, int64_t n)
+{
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= n) return;
+    const int side = (int)(t & 1), nx = a.nx, nr = a.nr, nc = nx - 1;
+    const int64_t lcol = t >> 1;
+    const int Y = (int)(lcol % nx), X = (int)((lcol / nx) % nx), sd = (int)(lcol / ((int64_t)nx * nx));
+    double acc = 0.0;
+    if (side == 0 ? a.sd_cmb[sd] != 0 : a.sd_surf[sd] != 0) {
+        const int rc = side == 0 ? 0 : nr - 2;
+        const double r1 = a.radii[(int64_t)sd * nr + rc], r2 = a.radii[(int64_t)sd * nr + rc + 1];
+        for (int k = 0; k < 4; ++k) {
+            const int xc = X - (k & 1), yc = Y - (k >> 1);
+            if (xc < 0 || xc >= nc || yc < 0 || yc >= nc) continue;
+            const int64_t col = ((int64_t)sd * nc + xc) * nc + yc;
+            for (int w = 0; w < 2; ++w) {
+                // wedge corners as corner columns of the cell; the node is corner k
+                const int kc = w == 0 ? (k == 3 ? -1 : k) : (k == 0 ? -1 : 3 - k);
+                if (kc < 0) continue;
+                SupgGeom G;
+                for (int s = 0; s < 3; ++s) supg_geometry(a, col, w, s, G);
+                double ub[3][4], ut[3][4], db[3], dt_[3];
+                for (int j = 0; j < 3; ++j) {
+                    const int64_t i = (((int64_t)sd * nx + xc + kEW[w][j][0]) * nx + yc + kEW[w][j][1]) * nr + rc;
+                    ub[0][j] = a.u0[i];
+                    ub[1][j] = a.u1[i];
+                    ub[2][j] = a.u2[i];
+                    ut[0][j] = a.u0[i + 1];
+                    ut[1][j] = a.u1[i + 1];
+                    ut[2][j] = a.u2[i + 1];
+                }
+                const double tau = a.tau ? a.tau[2 * ((col << a.lr) + rc) + w] : 0.0;
+                supg_wedge_diag(a, &G, 0, ub, ut, r1, r2, tau, db, dt_);
+                double mb = 0.0, mt = 0.0;
+                if (a.lumped) supg_lumped_mass(a, G, r1, r2, mb, mt);
+                const double vb = kc == 0 ? db[0] : (kc == 1 ? db[1] : db[2]);
+                const double vt = kc == 0 ? dt_[0] : (kc == 1 ? dt_[1] : dt_[2]);
+                acc += side == 0 ? vb + mb : vt + mt;
+            }
+        }
+    }
+    bdiag[t] = acc;
 }
 
 // g: the Dirichlet temperatures at the boundary nodes (CMB first), zero elsewhere
@@ -219,37 +565,107 @@ unsigned grid1d(int64_t n) { return (unsigned)((n + 255) / 256); }
 
 }  // namespace
 
-void supg_apply(tng_operator &op, const tng_vector &src, tng_vector &dst, hipStream_t s)
+namespace {
+
+int log2_of(int v)
+{
+    int l = 0;
+    while ((1 << l) < v) ++l;
+    TNG_REQUIRE((1 << l) == v, "SUPG: cells per subdomain must be a power of 2");
+    return l;
+}
+
+// cells of one block of the cell kernel: a radial segment of up to 256 cells,
+// or up to 64 whole columns (the lateral data of each sits in LDS)
+int supg_block(int ncr) { return std::min(256, 64 * ncr); }
+
+SupgArgs supg_args(const tng_operator &op)
 {
     const tng_domain &m = *op.mesh;
     TNG_REQUIRE(op.vel && op.vel->mesh == &m && op.vel->ncomp == 3 && op.vel->dtype == TNG_F64,
                 "SUPG: the velocity must be an FP64 vector on the operator's mesh");
-    TNG_REQUIRE(src.dtype == TNG_F64 && m.nr >= 2, "SUPG: FP64 temperature");
-    const int64_t ncell = (int64_t)m.nsd * (m.nx - 1) * (m.nx - 1) * (m.nr - 1);
-    const size_t bytes = (size_t)ncell * 12 * sizeof(double);
-    if (op.scratch.bytes < bytes) op.scratch.alloc(bytes);
     SupgArgs a{};
-    a.src = (const double *)src.comp(0);
     a.u0 = (const double *)op.vel->comp(0);
     a.u1 = (const double *)op.vel->comp(1);
     a.u2 = (const double *)op.vel->comp(2);
     a.coords = m.d_coords.as<double>();
     a.radii = m.d_radii.as<double>();
-    a.bmask = m.d_bmask.as<uint8_t>();
-    a.partial = op.scratch.as<double>();
+    a.sd_cmb = m.d_sd_cmb.as<uint8_t>();
+    a.sd_surf = m.d_sd_surf.as<uint8_t>();
     a.kappa = op.supg_kappa;
     a.dt = op.supg_dt;
     a.mass = op.supg_mass_scaling;
     a.treat_boundary = op.supg_treat_boundary ? 1 : 0;
-    a.diagonal = op.diagonal ? 1 : 0;
     a.lumped = op.supg_lumped ? 1 : 0;
-    a.supg = op.supg_enabled ? 1 : 0;
     a.nsd = m.nsd;
     a.nx = m.nx;
     a.nr = m.nr;
-    hipLaunchKernelGGL(supg_cell_kernel, dim3((unsigned)((ncell + 127) / 128)), dim3(128), 0, s, a);
+    a.lr = log2_of(m.nr - 1);
+    a.lc = log2_of(m.nx - 1);
+    a.lseg = std::min(a.lr, 8);
+    a.plen = m.nr + ((1 << a.lr) >> a.lseg) - 1;
+    a.ncell = (int64_t)m.nsd << (2 * a.lc + a.lr);
+    TNG_REQUIRE(a.ncell < (int64_t)1 << 31, "SUPG: cells exceed 32-bit indexing");
+    return a;
+}
+
+}  // namespace
+
+void supg_tau(const tng_operator &op, double *tau, hipStream_t s)
+{
+    const SupgArgs a = supg_args(op);
+    hipLaunchKernelGGL(supg_tau_kernel, dim3(grid1d(a.ncell)), dim3(256), 0, s, a, tau);
     TNG_HIP_CHECK(hipGetLastError());
-    launch_wedge_gather(op.scratch.as<double>(), dst, op.apply_mode == TNG_ADD, s);
+}
+
+void supg_boundary_diagonal(const tng_operator &op, const double *tau, double *bdiag, hipStream_t s)
+{
+    SupgArgs a = supg_args(op);
+    a.tau = op.supg_enabled ? tau : nullptr;
+    const int64_t n = 2 * op.mesh->nlat;
+    hipLaunchKernelGGL(supg_bdiag_kernel, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, s, a, bdiag, n);
+    TNG_HIP_CHECK(hipGetLastError());
+}
+
+size_t supg_tau_count(const tng_domain &m) { return (size_t)m.nsd * (m.nx - 1) * (m.nx - 1) * (m.nr - 1) * 2; }
+
+void supg_apply(tng_operator &op, const tng_vector &src, tng_vector &dst, hipStream_t s)
+{
+    const tng_domain &m = *op.mesh;
+    TNG_REQUIRE(src.dtype == TNG_F64 && m.nr >= 2, "SUPG: FP64 temperature");
+    SupgArgs a = supg_args(op);
+    // work space: corner partials, then (outside an energy step, which brings
+    // its own) tau and the boundary diagonal of this apply's velocity
+    const size_t npart = (size_t)(a.ncell >> a.lr) * 4 * a.plen, ntau = supg_tau_count(m), nb = 2 * (size_t)m.nlat;
+    const bool own_tau = op.supg_enabled && !op.supg_step_tau;
+    const bool treat = op.supg_treat_boundary && !op.diagonal;
+    const bool own_bdiag = treat && !op.supg_step_bdiag;
+    const size_t bytes = (npart + (own_tau ? ntau : 0) + (own_bdiag ? nb : 0)) * sizeof(double);
+    if (op.scratch.bytes < bytes) op.scratch.alloc(bytes);
+    a.src = (const double *)src.comp(0);
+    a.dst = (double *)dst.comp(0);
+    a.partial = op.scratch.as<double>();
+    a.add = op.apply_mode == TNG_ADD ? 1 : 0;
+    if (op.supg_enabled) {
+        if (own_tau) supg_tau(op, a.partial + npart, s);
+        a.tau = own_tau ? a.partial + npart : op.supg_step_tau;
+    }
+    if (treat) {
+        double *own = a.partial + npart + (own_tau ? ntau : 0);
+        if (own_bdiag) supg_boundary_diagonal(op, a.tau, own, s);
+        a.bdiag = own_bdiag ? own : op.supg_step_bdiag;
+    }
+    const int tb = supg_block(1 << a.lr), cols = std::max(1, tb >> a.lr);
+    const size_t lds = (size_t)cols * 2 * sizeof(SupgGeom) + (size_t)tb * 4 * sizeof(double);
+    const dim3 grid((unsigned)((a.ncell + tb - 1) / tb));
+    if (op.diagonal) {
+        a.treat_boundary = 0;  // every row keeps its own diagonal entry
+        hipLaunchKernelGGL(supg_cell_kernel<true>, grid, dim3(tb), lds, s, a);
+    } else {
+        hipLaunchKernelGGL(supg_cell_kernel<false>, grid, dim3(tb), lds, s, a);
+    }
+    hipLaunchKernelGGL(supg_gather_kernel, dim3(grid1d(m.nalloc)), dim3(256), 0, s, a, Index4(m.nx, m.nr));
+    TNG_HIP_CHECK(hipGetLastError());
     if (op.comm_mode == TNG_COMMUNICATE_ADDITIVELY) launch_halo_sum(m, dst, s);
 }
 

@@ -1554,15 +1554,6 @@ void launch_scalar_mass(const tng_vector &src, tng_vector &dst, hipStream_t s)
     launch_halo_sum(m, dst, s);
 }
 
-// Node sums of per-cell wedge partials (cell, wedge, 6 wedge nodes), FP64 scalar.
-void launch_wedge_gather(const double *partial, tng_vector &dst, bool add, hipStream_t s)
-{
-    const tng_domain &m = *dst.mesh;
-    hipLaunchKernelGGL(wedge_gather_kernel<double>, dim3(blocks_for(m.nalloc)), dim3(256), 0, s, partial,
-                       (double *)dst.comp(0), add ? 1 : 0, m.nsd, m.nx, m.nr, Index4(m.nx, m.nr));
-    TNG_HIP_CHECK(hipGetLastError());
-}
-
 }  // namespace tng
 
 // ----------------------------------------------------------------------------

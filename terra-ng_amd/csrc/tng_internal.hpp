@@ -269,6 +269,9 @@ struct tng_operator {
     tng_vector *vel = nullptr;
     double supg_kappa = 0.0, supg_dt = 0.0, supg_mass_scaling = 1.0;
     bool supg_treat_boundary = true, supg_lumped = false, supg_enabled = true;
+    // tau and boundary diagonal of the velocity at hand, set for the duration of
+    // one energy step only (nullptr: every apply computes its own)
+    const double *supg_step_tau = nullptr, *supg_step_bdiag = nullptr;
     // stored local matrices (OperatorStoredMatrixMode::Full): (sd, xc, yc, rc, wedge, 18, 18)
     bool stored = false;
     tng_dtype lmat_dtype = TNG_F64;
@@ -364,8 +367,10 @@ void stored_apply(tng_operator &op, const tng_vector &src, tng_vector &dst, cons
 
 // energy equation (kernels_energy.hip, kernels_stokes.hip)
 void supg_apply(tng_operator &op, const tng_vector &src, tng_vector &dst, hipStream_t s);
+size_t supg_tau_count(const tng_domain &m);  // one tau per wedge
+void supg_tau(const tng_operator &op, double *tau, hipStream_t s);
+void supg_boundary_diagonal(const tng_operator &op, const double *tau, double *bdiag, hipStream_t s);  // 2 nlat
 void launch_scalar_mass(const tng_vector &src, tng_vector &dst, hipStream_t s);
-void launch_wedge_gather(const double *partial, tng_vector &dst, bool add, hipStream_t s);
 void launch_boundary_values(tng_vector &g, double t_cmb, double t_surf, hipStream_t s);
 void launch_assign_masked(tng_vector &b, const tng_vector &src, uint8_t flag, hipStream_t s);
 void launch_viscosity_fk(tng_vector &eta, const tng_vector &temp, double rmu, hipStream_t s);

@@ -1,0 +1,51 @@
+"""Kernel variants at the sizes where their decompositions change: against
+the oracle at 1e-12 (FP64: sums of at most a few hundred products of one
+sign-free magnitude, 1e-16 each)."""
+import numpy as np
+import pytest
+
+import oracle as O
+import tng
+from conftest import consistent, rel_err
+
+pytestmark = pytest.mark.gpu
+
+D, F = tng.DIRICHLET, tng.FREESLIP
+
+
+def field(om, ncomp, seed, scale=1.0):
+    r = np.random.default_rng(seed)
+    return consistent(om, scale * r.uniform(-1, 1, ((ncomp,) if ncomp > 1 else ()) + om.shape))
+
+
+def vec(dom, data, dtype=tng.F64):
+    return (tng.VectorQ1Vec if data.ndim == 5 else tng.VectorQ1Scalar)(dom, dtype).upload(data)
+
+
+# columns per block of the SUPG cell kernel: 64 (2 and 4 cells), 32, one, and
+# radial segments of 256 cells whose seam levels two blocks share (512 layers)
+@pytest.mark.parametrize("L,Lr,ls,rs", [(2, 1, 0, 0), (3, 2, 1, 0), (2, 3, 0, 0), (2, 8, 0, 0), (1, 9, 0, 0), (1, 9, 0, 1)])
+@pytest.mark.parametrize("flags", [dict(), dict(lumped_mass=True), dict(diagonal=True, treat_boundary=False)])
+def test_supg_block_shapes(L, Lr, ls, rs, flags, gpu_ctx):
+    dom = tng.DistributedDomain.create_uniform(L, Lr, 0.55, 1.0, ls, rs)
+    om = O.Mesh(L, Lr, 0.55, 1.0, ls, rs)
+    vel, T = field(om, 3, 1, 50.0), field(om, 1, 2)
+    op = tng.UnsteadyAdvectionDiffusionSUPG(dom, vec(dom, vel), 0.01, 0.02, **flags)
+    out = vec(dom, T)
+    op.apply(vec(dom, T), out)
+    ref = O.supg_apply(om, vel, T, kappa=0.01, dt=0.02, treat_boundary=flags.get("treat_boundary", True),
+                       diagonal=flags.get("diagonal", False), lumped=flags.get("lumped_mass", False))
+    assert rel_err(out.download(), ref) < 1e-12
+
+
+def test_supg_reads_the_velocity_at_every_apply(gpu_ctx):
+    """tau and the boundary rows follow a velocity changed in place between two applies of one operator."""
+    dom, om = tng.DistributedDomain.create_uniform(3, 3, 0.55, 1.0), O.Mesh(3)
+    T, v = field(om, 1, 2), vec(dom, field(om, 3, 1, 50.0))
+    op = tng.UnsteadyAdvectionDiffusionSUPG(dom, v, 0.01, 0.02)
+    out = vec(dom, T)
+    op.apply(vec(dom, T), out)
+    vel = field(om, 3, 3, 5.0)
+    v.upload(vel)
+    op.apply(vec(dom, T), out)
+    assert rel_err(out.download(), O.supg_apply(om, vel, T, kappa=0.01, dt=0.02)) < 1e-12
