@@ -49,3 +49,18 @@ def test_supg_reads_the_velocity_at_every_apply(gpu_ctx):
     v.upload(vel)
     op.apply(vec(dom, T), out)
     assert rel_err(out.download(), O.supg_apply(om, vel, T, kappa=0.01, dt=0.02)) < 1e-12
+
+
+# rows at every kind of node: subdomain edges and corners, single cells between surfaces, 128 layers
+@pytest.mark.parametrize("L,Lr,ls,rs", [(1, 1, 0, 0), (2, 3, 1, 1), (3, 2, 0, 0), (2, 7, 0, 0)])
+def test_mass_matches_oracle(L, Lr, ls, rs, gpu_ctx):
+    dom = tng.DistributedDomain.create_uniform(L, Lr, 0.55, 1.0, ls, rs)
+    om = O.Mesh(L, Lr, 0.55, 1.0, ls, rs)
+    x, u = field(om, 1, 4), field(om, 3, 5)
+    out = vec(dom, x)
+    tng.mass_apply(vec(dom, x), out)
+    assert rel_err(out.download(), O.scalar_mass(om, x)) < 1e-12
+    for dtype, tol in ((tng.F64, 1e-12), (tng.F32, 2e-6)):  # FP32: inputs and tables rounded to 6e-8, sums of 63 terms
+        out = vec(dom, u, dtype)
+        tng.VectorMass(dom).apply(vec(dom, u, dtype), out)
+        assert rel_err(out.download(), O.vector_mass(om, u)) < tol
