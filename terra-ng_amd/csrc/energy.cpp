@@ -31,8 +31,10 @@ struct tng_energy_s {
     tng_vector *vel = nullptr, *temp = nullptr;
     std::unique_ptr<tng_operator> A, A_neumann, A_neumann_diag;
     std::vector<std::unique_ptr<tng_vector>> pool;
-    tng_vector *g = nullptr, *tmp = nullptr, *q = nullptr, *diag = nullptr, *ones = nullptr, *t_backup = nullptr;
+    tng_vector *g = nullptr, *tmp = nullptr, *q = nullptr, *diag = nullptr, *diag_raw = nullptr,
+               *ones = nullptr, *t_backup = nullptr;
     std::vector<tng_vector *> fg;  // FGMRES work space: 2m + 4 scalars
+    tng::DevBuf h_dev;             // the projections of an Arnoldi step
     tng::DevBuf tau, bdiag;        // SUPG tau per wedge and boundary diagonal of the step's velocity
     double h = 0.0;
 };
@@ -101,7 +103,10 @@ void energy_fgmres(tng_energy_s &e, tng_operator &A, tng_vector &x, const tng_ve
         return;
     }
     const int offV = 1, offZ = offV + m + 1, idxW = offZ + m, idxAcc = idxW + 1;
-    std::vector<double> H((size_t)(m + 1) * m), g(m + 1), cs(m + 1), sn(m + 1), y;
+    std::vector<double> H((size_t)(m + 1) * m), g(m + 1), cs(m + 1), sn(m + 1), y, hcol(m + 2);
+    if (e.h_dev.bytes < (m + 2) * sizeof(double)) e.h_dev.alloc((m + 2) * sizeof(double));
+    double *hdev = e.h_dev.as<double>();
+    hipStream_t s = stream_of(x);
     auto h = [&](int i, int j) -> double & { return H[(size_t)i * m + j]; };
     int total = 0;
     while (total < e.prm.krylov_max_iterations) {
@@ -113,14 +118,17 @@ void energy_fgmres(tng_energy_s &e, tng_operator &A, tng_vector &x, const tng_ve
         for (int j = 0; j < m && total < e.prm.krylov_max_iterations; ++j, ++total) {
             tng_vector &vj = *e.fg[offV + j], &zj = *e.fg[offZ + j], &w = *e.fg[idxW];
             rep.iterations += 1;
-            launch_copy(zj, vj, stream_of(zj));
-            launch_mult(zj, *e.diag, stream_of(zj));
+            launch_diag_mult(zj, *e.diag, vj, s);
             op_apply(A, zj, w);
-            for (int i = 0; i <= j; ++i) {
-                h(i, j) = dot(w, *e.fg[offV + i]);
-                lincomb(w, {1.0, -h(i, j)}, {&w, e.fg[offV + i]});
-            }
-            const double hj1 = std::sqrt(dot(w, w));
+            // one fused pass per basis vector (axpy with the coefficient before,
+            // next dot), the coefficients on the device, one copy per step
+            for (int i = 0; i <= j + 1; ++i)
+                launch_mgs_step(w, nullptr, i > 0 ? e.fg[offV + i - 1] : nullptr, nullptr,
+                                i > 0 ? hdev + i - 1 : nullptr, i <= j ? e.fg[offV + i] : nullptr, nullptr, hdev + i, s);
+            TNG_HIP_CHECK(hipMemcpyAsync(hcol.data(), hdev, sizeof(double) * (j + 2), hipMemcpyDeviceToHost, s));
+            TNG_HIP_CHECK(hipStreamSynchronize(s));
+            for (int i = 0; i <= j; ++i) h(i, j) = hcol[i];
+            const double hj1 = std::sqrt(hcol[j + 1]);
             if (hj1 < std::numeric_limits<double>::epsilon() * initial) {
                 h(j + 1, j) = 0;
                 inner = j + 1;
@@ -161,9 +169,9 @@ void energy_fgmres(tng_energy_s &e, tng_operator &A, tng_vector &x, const tng_ve
         }
         y.assign(inner, 0.0);
         for (int row = inner - 1; row >= 0; --row) {
-            double s = g[row];
-            for (int col = row + 1; col < inner; ++col) s -= h(row, col) * y[col];
-            y[row] = s / h(row, row);
+            double sum = g[row];
+            for (int col = row + 1; col < inner; ++col) sum -= h(row, col) * y[col];
+            y[row] = sum / h(row, row);
         }
         tng_vector &acc = *e.fg[idxAcc];
         launch_fill(acc, 0.0, stream_of(acc));
@@ -230,7 +238,8 @@ void energy_step(tng_energy_s &e, double dt, tng_solve_report &rep)
     supg_tau(*e.A, e.tau.as<double>(), s);
     supg_boundary_diagonal(*e.A, e.tau.as<double>(), e.bdiag.as<double>(), s);
     // inverse diagonal at the step's dt
-    op_apply(*e.A_neumann_diag, *e.ones, *e.diag);
+    op_apply(*e.A_neumann_diag, *e.ones, *e.diag_raw);
+    launch_copy(*e.diag, *e.diag_raw, s);
     launch_invert(*e.diag, s);
     reset_report(rep);
     for (int i = 0; i < e.prm.energy_substeps; ++i) {
@@ -238,7 +247,7 @@ void energy_step(tng_energy_s &e, double dt, tng_solve_report &rep)
         launch_boundary_values(*e.g, e.prm.temperature_cmb, e.prm.temperature_surface, s);
         op_apply(*e.A_neumann, *e.g, *e.tmp);                                   // g_A = A_N g
         lincomb(*e.q, {1.0, -1.0}, {e.q, e.tmp});                               // q -= g_A
-        op_apply(*e.A_neumann_diag, *e.g, *e.tmp);                              // g_D = diag(A_N) g
+        launch_diag_mult(*e.tmp, *e.diag_raw, *e.g, s);                         // g_D = diag(A_N) g
         launch_assign_masked(*e.q, *e.tmp, SBF_BOUNDARY, s);                    // q = g_D on the boundary
         tng_solve_report sub{};
         sub.history = rep.history ? rep.history + std::min(rep.history_len, rep.history_capacity) : nullptr;
@@ -361,6 +370,7 @@ tng_status tng_energy_create(tng_stokes_solver solver, tng_vec velocity, tng_vec
         e->tmp = evec(*e, m);
         e->q = evec(*e, m);
         e->diag = evec(*e, m);
+        e->diag_raw = evec(*e, m);
         e->ones = evec(*e, m);
         e->t_backup = evec(*e, m);
         launch_fill(*e->ones, 1.0, m->ctx->stream);

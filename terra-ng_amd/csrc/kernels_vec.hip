@@ -282,6 +282,26 @@ template <typename T> __global__ __launch_bounds__(256) void mult_kernel(const C
         for (int c = 0; c < ncomp; ++c) y.p[c][i] *= x.p[c][i];
 }
 
+// z = d * x entrywise (the Jacobi preconditioner): one pass instead of a copy
+// and an in-place product.
+template <typename T, int V>
+__global__ __launch_bounds__(256) void diag_mult_kernel(const Comp3<T> z, const Comp3<T> d, const Comp3<T> x, int ncomp,
+                                                        int64_t n)
+{
+    const int64_t t0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (int64_t)gridDim.x * blockDim.x;
+    for (int c = 0; c < ncomp; ++c) {
+        for (int64_t i = t0; i < n / V; i += stride) {
+            Pack<T, V> a = ldv<V>(x.p[c], i);
+            const Pack<T, V> b = ldv<V>(d.p[c], i);
+#pragma unroll
+            for (int k = 0; k < V; ++k) a.e[k] *= b.e[k];
+            stv<V>(z.p[c], i, a);
+        }
+        if constexpr (V > 1)
+            for (int64_t i = n / V * V + t0; i < n; i += stride) z.p[c][i] = x.p[c][i] * d.p[c][i];
+    }
+}
+
 // One Chebyshev sub-step (linalg/solvers/chebyshev.hpp:102-165) in one pass:
 //   z = invd * (b - Ax)   (Ax absent: x = 0)
 //   d = cz * z + cd * d   (cd absent: d is overwritten)
@@ -639,6 +659,28 @@ void launch_mult(tng_vector &y, const tng_vector &x, hipStream_t s)
     TNG_HIP_CHECK(hipGetLastError());
 }
 
+void launch_diag_mult(tng_vector &z, const tng_vector &d, const tng_vector &x, hipStream_t s)
+{
+    TNG_REQUIRE(x.mesh == z.mesh && d.mesh == z.mesh && x.dtype == z.dtype && d.dtype == z.dtype &&
+                    x.ncomp == z.ncomp && d.ncomp == z.ncomp,
+                "diagonal product: mismatched vectors");
+    const int64_t n = z.mesh->nalloc;
+    const int nc = z.ncomp;
+    auto run = [&](auto tag) {
+        using T = decltype(tag);
+        const Comp3<T> pz = comps<T>(z), pd = comps<T>(d), px = comps<T>(x);
+        if (aligned16(pz, nc) && aligned16(pd, nc) && aligned16(px, nc))
+            hipLaunchKernelGGL((diag_mult_kernel<T, kVec<T>>), dim3(gs(n / kVec<T>)), dim3(256), 0, s, pz, pd, px, nc, n);
+        else
+            hipLaunchKernelGGL((diag_mult_kernel<T, 1>), dim3(gs(n)), dim3(256), 0, s, pz, pd, px, nc, n);
+    };
+    if (z.dtype == TNG_F64)
+        run(double());
+    else
+        run(float());
+    TNG_HIP_CHECK(hipGetLastError());
+}
+
 void launch_cheb_update(tng_vector &x, tng_vector &d, const tng_vector &b, const tng_vector *ax,
                         const tng_vector &invd, double cz, double cd, bool read_d, bool x_zero, hipStream_t s)
 {
@@ -787,17 +829,19 @@ void launch_pcg_direction(tng_vector &p, const tng_vector &r, hipStream_t s)
     TNG_HIP_CHECK(hipGetLastError());
 }
 
-// MGS step on a Stokes vector (u, p): h_out = (w -= h_prev v_prev) . v_next
-void launch_mgs_step(tng_vector &wu, tng_vector &wp, const tng_vector *vprev_u, const tng_vector *vprev_p,
+// MGS step on a vector (u, p), p absent (nullptr) for a single field:
+// h_out = (w -= h_prev v_prev) . v_next
+void launch_mgs_step(tng_vector &wu, tng_vector *wp, const tng_vector *vprev_u, const tng_vector *vprev_p,
                      const double *h_prev_dev, const tng_vector *vnext_u, const tng_vector *vnext_p, double *h_out_dev,
                      hipStream_t s)
 {
     tng_context &ctx = *wu.mesh->ctx;
     double *part = ctx.red_partials.as<double>();
     unsigned g[2] = {0, 0};
-    tng_vector *w[2] = {&wu, &wp};
+    tng_vector *w[2] = {&wu, wp};
     const tng_vector *vp[2] = {vprev_u, vprev_p}, *vn[2] = {vnext_u, vnext_p};
     for (int b = 0; b < 2; ++b) {
+        if (!w[b]) continue;
         const tng_vector &wb = *w[b];
         const int64_t n = wb.mesh->nalloc;
         const tng_vector &pv = vp[b] ? *vp[b] : wb, &nv = vn[b] ? *vn[b] : wb;

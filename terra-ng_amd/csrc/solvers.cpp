@@ -702,7 +702,7 @@ void StokesSolver::fgmres(SVec &x, const SVec &b, tng_solve_report &rep)
             for (int i = 0; i <= j + 1; ++i) {
                 const SVec *vprev = i > 0 ? &fg[offV + i - 1] : nullptr;
                 const SVec *vnext = i <= j ? &fg[offV + i] : nullptr;
-                launch_mgs_step(*w.u, *w.p, vprev ? vprev->u : nullptr, vprev ? vprev->p : nullptr,
+                launch_mgs_step(*w.u, w.p, vprev ? vprev->u : nullptr, vprev ? vprev->p : nullptr,
                                 i > 0 ? hdev + i - 1 : nullptr, vnext ? vnext->u : nullptr,
                                 vnext ? vnext->p : nullptr, hdev + i, stream_of(*w.u));
             }

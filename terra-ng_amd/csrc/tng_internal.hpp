@@ -318,6 +318,7 @@ void stokes_block_apply(tng_operator &op, const tng_vector &src, tng_vector &dst
 // BLAS-1 and reductions (kernels_vec.hip)
 void launch_lincomb(tng_vector &y, int nx, const double *c, const tng_vector *const *x, double c0, hipStream_t s);
 void launch_mult(tng_vector &y, const tng_vector &x, hipStream_t s);
+void launch_diag_mult(tng_vector &z, const tng_vector &d, const tng_vector &x, hipStream_t s);  // z = d x
 void launch_invert(tng_vector &y, hipStream_t s);
 void launch_cheb_update(tng_vector &x, tng_vector &d, const tng_vector &b, const tng_vector *ax,
                         const tng_vector &invd, double cz, double cd, bool read_d, bool x_zero, hipStream_t s);
@@ -331,8 +332,9 @@ void launch_pcg_update(tng_vector &x, tng_vector &r, const tng_vector &p, const 
                        double atol, int it, hipStream_t s);
 void launch_pcg_direction(tng_vector &p, const tng_vector &r, hipStream_t s);
 void pcg_read_state(const tng_vector &v, int *done, int *iters, double *final_rel, hipStream_t s);
-// FGMRES modified Gram-Schmidt step on a Stokes vector; h values live on the device
-void launch_mgs_step(tng_vector &wu, tng_vector &wp, const tng_vector *vprev_u, const tng_vector *vprev_p,
+// FGMRES modified Gram-Schmidt step on a vector (wp and its partners nullptr:
+// one field); h values live on the device
+void launch_mgs_step(tng_vector &wu, tng_vector *wp, const tng_vector *vprev_u, const tng_vector *vprev_p,
                      const double *h_prev_dev, const tng_vector *vnext_u, const tng_vector *vnext_p, double *h_out_dev,
                      hipStream_t s);
 double *device_slots(tng_context &ctx, int first);  // ctx.red_result + first (doubles, 512 in total)
