@@ -7,6 +7,7 @@
 //
 //   unique numbering: uid[copy] = unique node of a node copy; rep[node] = one
 //   copy of it.  Unknown 3 u + c is component c of unique node u.
+#include <cfloat>
 #include <cmath>
 #include <string>
 #include <vector>
@@ -151,10 +152,15 @@ unsigned blocks(int64_t n) { return (unsigned)((n + 255) / 256); }
 
 }  // namespace
 
-void CoarseDirect::numbering(const tng_domain &m)
+namespace {
+
+// uid[copy] = unique node of a node copy, rep[node] = its first copy
+void number_nodes(const tng_domain &m, std::vector<int32_t> &uid, std::vector<int32_t> &rep)
 {
     const int64_t nc = m.nalloc;
-    std::vector<int32_t> uid(nc), hidx((size_t)m.halo_maxc * m.halo_n);
+    std::vector<int32_t> hidx((size_t)m.halo_maxc * m.halo_n);
+    uid.resize(nc);
+    rep.clear();
     if (!hidx.empty())
         TNG_HIP_CHECK(hipMemcpy(hidx.data(), m.d_halo_idx.p, hidx.size() * sizeof(int32_t), hipMemcpyDeviceToHost));
     for (int64_t i = 0; i < nc; ++i) uid[i] = (int32_t)i;
@@ -166,22 +172,34 @@ void CoarseDirect::numbering(const tng_domain &m)
             if (c >= 0) uid[c] = first;
         }
     }
-    std::vector<int32_t> compact(nc, -1), rep;
+    std::vector<int32_t> compact(nc, -1);
     for (int64_t i = 0; i < nc; ++i)
         if (uid[i] == i) {
             compact[i] = (int32_t)rep.size();
             rep.push_back((int32_t)i);
         }
     for (int64_t i = 0; i < nc; ++i) uid[i] = compact[uid[i]];
+}
+
+void upload(DevBuf &b, const void *src, size_t bytes)
+{
+    b.alloc(bytes);
+    TNG_HIP_CHECK(hipMemcpy(b.p, src, bytes, hipMemcpyHostToDevice));
+}
+
+}  // namespace
+
+void CoarseDirect::numbering(const tng_domain &m)
+{
+    std::vector<int32_t> uid, rep;
+    number_nodes(m, uid, rep);
     nu = (int)rep.size();
     n = 3 * nu;
     TNG_REQUIRE(n <= kMaxUnknowns, "direct coarse solve: the coarsest level has " + std::to_string(n) +
                                        " unknowns, more than " + std::to_string(kMaxUnknowns));
-    ncopies = nc;
-    d_uid.alloc(nc * sizeof(int32_t));
-    d_rep.alloc(rep.size() * sizeof(int32_t));
-    TNG_HIP_CHECK(hipMemcpy(d_uid.p, uid.data(), nc * sizeof(int32_t), hipMemcpyHostToDevice));
-    TNG_HIP_CHECK(hipMemcpy(d_rep.p, rep.data(), rep.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+    ncopies = m.nalloc;
+    upload(d_uid, uid.data(), uid.size() * sizeof(int32_t));
+    upload(d_rep, rep.data(), rep.size() * sizeof(int32_t));
     d_M.alloc((size_t)n * n * sizeof(double));
     d_row.alloc(n * sizeof(double));
     d_col.alloc(n * sizeof(double));
@@ -316,6 +334,397 @@ void CoarseDirect::solve(tng_vector &e0, const tng_vector &r0, hipStream_t s)
         hipLaunchKernelGGL(scatter_kernel<float>, dim3(blocks(ncopies)), dim3(256), 0, s, (float *)e0.comp(0),
                            (float *)e0.comp(1), (float *)e0.comp(2), uid, ncopies, (const double *)x);
     TNG_HIP_CHECK(hipGetLastError());
+}
+
+// ----------------------------------------------------------------------------
+// PCG on the assembled coarsest operator.  A coarsest level has a few hundred
+// to a few thousand nodes: its PCG is bound by launches and by the chain of
+// loads in each kernel, not by bandwidth.  Assembled over the unique nodes the
+// halo sum and the boundary handling are in the matrix (1.2 MB at level 2
+// against 3.3 MB of wedge matrices, most of which five blocks of gathering
+// threads read per apply), and each of an iteration's two reductions ends in
+// the next kernel, where every block sums the partials itself.  Level 2 (810
+// nodes), Galerkin operator: 8.8 us per iteration (5.2 + 3.6), 71 us with the
+// stored-matrix apply, halo sum and five vector kernels.  Used up to 8192
+// nodes (lateral level 3), where the matrix kernel's 10 MB still come from
+// cache; above, and with the rotation penalty (a rank-3 term over all nodes),
+// the general PCG on the operator's own apply runs.
+// ----------------------------------------------------------------------------
+namespace {
+
+// The wedge (dxc, dyc, w, rc) around a node copy (X, Y, l), q = 0 .. 11, as the
+// lateral cell offsets, the wedge, the radial cell offset and the node's
+// lateral corner in it.
+__host__ __device__ __forceinline__ void wedge_around(int q, int &dx, int &dy, int &w, int &dr, int &corner)
+{
+    // lateral triangles around a node: cell offsets, wedge, corner
+    constexpr int8_t kT[6][4] = {{0, 0, 0, 0}, {-1, 0, 1, 2}, {-1, 0, 0, 1}, {-1, -1, 1, 0}, {0, -1, 0, 2}, {0, -1, 1, 1}};
+    const int t = q >> 1;
+    dr = (q & 1) - 1;
+    dx = kT[t][0];
+    dy = kT[t][1];
+    w = kT[t][2];
+    corner = kT[t][3];
+}
+
+struct CpcgArgs {
+    const double *lmat;
+    const int32_t *rep, *copy_begin, *copy_list;
+    const uint8_t *slot;
+    const double *coords;
+    const uint8_t *sd_cmb, *sd_surf;
+    double *A;  // (node, entry 9, slot)
+    const int32_t *col;
+    int nu, nx, nr, bc_cmb, bc_surf;
+};
+
+// Sum of the wedge matrices' 3 x 3 blocks into the row's slots; one thread per
+// (node, entry), which owns that entry of every slot of the row.
+__global__ __launch_bounds__(64) void cpcg_assemble_kernel(const CpcgArgs a)
+{
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= a.nu * 9) return;
+    const int u = t / 9, e = t - 9 * u, d1 = e / 3, d2 = e - 3 * d1;
+    constexpr int W = CoarsePcg::kWidth;
+    double *row = a.A + ((int64_t)u * 9 + e) * W;
+    for (int s = 0; s < W; ++s) row[s] = 0.0;
+    const int nx = a.nx, nr = a.nr, nc = nx - 1, ncr = nr - 1;
+    for (int j = a.copy_begin[u]; j < a.copy_begin[u + 1]; ++j) {
+        const int i = a.copy_list[j];
+        const int l = i % nr, c = i / nr, Y = c % nx, X = (c / nx) % nx, sd = c / (nx * nx);
+        for (int q = 0; q < 12; ++q) {
+            int dx, dy, w, dr, corner;
+            wedge_around(q, dx, dy, w, dr, corner);
+            const int xc = X + dx, yc = Y + dy, rc = l + dr;
+            if (xc < 0 || xc >= nc || yc < 0 || yc >= nc || rc < 0 || rc >= ncr) continue;
+            const double *m = a.lmat + (((((int64_t)sd * nc + xc) * nc + yc) * ncr + rc) * 2 + w) * 324 +
+                              (corner + (dr == 0 ? 0 : 3) + 6 * d1) * 18 + 6 * d2;
+            const uint8_t *sl = a.slot + (int64_t)i * CoarsePcg::kMaxSlots + 6 * q;
+            for (int k = 0; k < 6; ++k) row[sl[k]] += m[k];
+        }
+    }
+}
+
+// kind of a node: 0 interior or Neumann, else its boundary condition; n its unit normal
+__device__ __forceinline__ int cpcg_node_bc(const CpcgArgs &a, int u, double n[3])
+{
+    const int i = a.rep[u], nx = a.nx, nr = a.nr, l = i % nr, c = i / nr, sd = c / (nx * nx);
+    const int bc = l == 0 && a.sd_cmb[sd] ? a.bc_cmb : (l == nr - 1 && a.sd_surf[sd] ? a.bc_surf : TNG_NEUMANN);
+    const double *q = a.coords + 3 * (int64_t)c;
+    const double mag = sqrt(q[0] * q[0] + q[1] * q[1] + q[2] * q[2]);
+    for (int d = 0; d < 3; ++d) n[d] = q[d] / mag;
+    return bc;
+}
+
+// Boundary rows and columns, per block: Dirichlet rows keep their diagonal
+// entries, Dirichlet columns vanish; free slip projects the normal component
+// out on both sides and keeps the normal-normal entry of the diagonal block.
+__global__ __launch_bounds__(64) void cpcg_boundary_kernel(const CpcgArgs a)
+{
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    constexpr int W = CoarsePcg::kWidth;
+    if (t >= a.nu * W) return;
+    const int u = t / W, s = t - W * u, v = a.col[t];
+    if (v < 0) return;
+    double nu_[3], nv[3], B[3][3];
+    const int bu = cpcg_node_bc(a, u, nu_), bv = cpcg_node_bc(a, v, nv);
+    double *row = a.A + (int64_t)u * 9 * W + s;
+    for (int e = 0; e < 9; ++e) B[e / 3][e % 3] = row[e * W];
+    if (bu == TNG_DIRICHLET || bv == TNG_DIRICHLET) {
+        for (int e = 0; e < 9; ++e) row[e * W] = u == v && bu == TNG_DIRICHLET && e % 4 == 0 ? B[e / 3][e / 3] : 0.0;
+        return;
+    }
+    if (bu != TNG_FREESLIP && bv != TNG_FREESLIP) return;
+    double ann = 0.0;
+    if (u == v)
+        for (int e = 0; e < 9; ++e) ann += nu_[e / 3] * B[e / 3][e % 3] * nu_[e % 3];
+    if (bv == TNG_FREESLIP)
+        for (int i = 0; i < 3; ++i) {
+            const double d = B[i][0] * nv[0] + B[i][1] * nv[1] + B[i][2] * nv[2];
+            for (int j = 0; j < 3; ++j) B[i][j] -= d * nv[j];
+        }
+    if (bu == TNG_FREESLIP)
+        for (int j = 0; j < 3; ++j) {
+            const double d = nu_[0] * B[0][j] + nu_[1] * B[1][j] + nu_[2] * B[2][j];
+            for (int i = 0; i < 3; ++i) B[i][j] -= d * nu_[i];
+        }
+    for (int e = 0; e < 9; ++e) row[e * W] = B[e / 3][e % 3] + (u == v ? ann * nu_[e / 3] * nu_[e % 3] : 0.0);
+}
+
+// state: iteration count, done flag, first residual norm, total iterations,
+// then r.r of iteration 0, 1, ... (kHist slots, used in turn)
+enum { CS_ITERS = 0, CS_DONE, CS_INIT, CS_TOTAL, CS_RR, CS_N = CS_RR + 2 };
+constexpr int kCpcgNodes = 16;    // nodes per block of the matrix kernel: 16 lanes each
+constexpr int kCpcgMaxParts = 1024;
+
+__device__ __forceinline__ double block_sum256(double v, double *red)
+{
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    const double s = (red[0] + red[1]) + (red[2] + red[3]);
+    __syncthreads();
+    return s;
+}
+__device__ __forceinline__ double parts_sum(const double *p, int n, double *red)
+{
+    double v = 0.0;
+    for (int i = threadIdx.x; i < n; i += 256) v += p[i];
+    return block_sum256(v, red);
+}
+
+// r = b, p = 0, x = 0; partials of r.r
+template <typename T>
+__global__ __launch_bounds__(256) void cpcg_begin_kernel(const Comp3<const T> b, const int32_t *rep, int nu, double *x,
+                                                         double *r, double *p, double *parts, double *st)
+{
+    __shared__ double red[4];
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    double v = 0.0;
+    if (t < 3 * nu) {
+        const int u = t / 3, c = t - 3 * u;
+        v = (double)(c == 0 ? b.p[0] : (c == 1 ? b.p[1] : b.p[2]))[rep[u]];
+        r[t] = v;
+        p[t] = 0.0;
+        x[t] = 0.0;
+    }
+    const double s = block_sum256(v * v, red);
+    if (threadIdx.x == 0) parts[blockIdx.x] = s;
+    if (t == 0) {
+        st[CS_ITERS] = 0.0;
+        st[CS_DONE] = 0.0;
+    }
+}
+
+// First kernel of iteration it (1, 2, ...): ends the iteration before (r.r, the
+// stopping test, beta), forms the direction p = r + beta p_old of the row's own
+// and neighbour nodes as it reads them, and A p with the partials of p.(A p).
+// Every block combines the partials in one fixed order, so all take the same
+// decision; block 0 records it.  16 lanes per row, lane j the slots j, j + 16.
+__global__ __launch_bounds__(256) void cpcg_matrix_kernel(const double *A, const int32_t *col, int nu, const double *r,
+                                                          const double *p_old, double *p, double *ap, const double *rparts,
+                                                          int nrp, double *pparts, double *st, int it, double rtol,
+                                                          double atol)
+{
+    __shared__ double red[4];
+    if (st[CS_DONE] != 0.0) return;  // written by an earlier launch
+    constexpr int W = CoarsePcg::kWidth;
+    const int u = blockIdx.x * kCpcgNodes + (threadIdx.x >> 4), lane = threadIdx.x & 15;
+    int v[2];
+    double B[2][9];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const int s = lane + 16 * k;
+        v[k] = u < nu && s < W ? col[u * W + s] : -1;
+#pragma unroll
+        for (int e = 0; e < 9; ++e) B[k][e] = v[k] >= 0 ? A[((int64_t)u * 9 + e) * W + s] : 0.0;
+    }
+    const double rr = parts_sum(rparts, nrp, red);
+    double beta = 0.0;
+    if (it == 1) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            const double init = sqrt(rr);
+            st[CS_INIT] = init;
+            st[CS_RR + 1] = rr;
+            if (init < atol) st[CS_DONE] = 1.0;
+        }
+        if (sqrt(rr) < atol) return;
+    } else {
+        const double rr_old = st[CS_RR + ((it - 1) & 1)], res = sqrt(rr);
+        const bool stop = res / st[CS_INIT] <= rtol || res < atol || fabs(rr_old) < DBL_MIN;
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            st[CS_RR + (it & 1)] = rr;
+            st[CS_ITERS] = it - 1;
+            if (stop) {
+                st[CS_DONE] = 1.0;
+                st[CS_TOTAL] += it - 1;
+            }
+        }
+        if (stop) return;
+        beta = rr / rr_old;
+    }
+    double y[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+        if (v[k] >= 0) {
+            double q[3];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) q[c] = fma(beta, p_old[3 * v[k] + c], r[3 * v[k] + c]);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) y[c] += B[k][3 * c] * q[0] + B[k][3 * c + 1] * q[1] + B[k][3 * c + 2] * q[2];
+        }
+    double d = 0.0;
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+        for (int o = 8; o > 0; o >>= 1) y[c] += __shfl_xor(y[c], o, 16);
+    if (u < nu && lane < 3) {
+        const double yc = lane == 0 ? y[0] : (lane == 1 ? y[1] : y[2]);
+        const double pc = fma(beta, p_old[3 * u + lane], r[3 * u + lane]);
+        p[3 * u + lane] = pc;
+        ap[3 * u + lane] = yc;
+        d = pc * yc;
+    }
+    const double s = block_sum256(d, red);
+    if (threadIdx.x == 0) pparts[blockIdx.x] = s;
+}
+
+// Second kernel: alpha, x += alpha p, r -= alpha A p, partials of r.r; the last
+// one allowed counts itself (no later kernel runs the test).
+__global__ __launch_bounds__(256) void cpcg_update_kernel(int n, double *x, double *r, const double *p, const double *ap,
+                                                          const double *pparts, int npp, double *rparts, double *st,
+                                                          int it, int max_it)
+{
+    __shared__ double red[4];
+    if (st[CS_DONE] != 0.0) return;
+    const double pap = parts_sum(pparts, npp, red);
+    const bool stop = fabs(pap) < DBL_MIN;
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t == 0 && (stop || it == max_it)) {
+        st[CS_ITERS] = it;
+        st[CS_TOTAL] += it;
+        if (stop) st[CS_DONE] = 1.0;
+    }
+    if (stop) return;
+    const double alpha = st[CS_RR + (it & 1)] / pap;
+    double rn = 0.0;
+    if (t < n) {
+        x[t] = fma(alpha, p[t], x[t]);
+        rn = fma(-alpha, ap[t], r[t]);
+        r[t] = rn;
+    }
+    const double s = block_sum256(rn * rn, red);
+    if (threadIdx.x == 0) rparts[blockIdx.x] = s;
+}
+
+}  // namespace
+
+bool CoarsePcg::accepts(const tng_operator &A)
+{
+    const tng_domain &m = *A.mesh;
+    return !A.penalty_active && m.nr >= 3 && m.num_owned <= kMaxNodes;
+}
+
+void CoarsePcg::numbering(const tng_domain &m)
+{
+    std::vector<int32_t> uid, rep;
+    number_nodes(m, uid, rep);
+    nu = (int)rep.size();
+    ncopies = m.nalloc;
+    const int nx = m.nx, nr = m.nr, nc = nx - 1, ncr = nr - 1;
+    std::vector<int32_t> begin(nu + 1, 0), list(ncopies), col((size_t)nu * kWidth, -1);
+    for (int64_t i = 0; i < ncopies; ++i) begin[uid[i] + 1]++;
+    for (int u = 0; u < nu; ++u) begin[u + 1] += begin[u];
+    std::vector<int32_t> at(begin.begin(), begin.end() - 1);
+    for (int64_t i = 0; i < ncopies; ++i) list[at[uid[i]]++] = (int32_t)i;
+    std::vector<uint8_t> slot((size_t)ncopies * kMaxSlots, 0);
+    static const int WN[2][3][2] = {{{0, 0}, {1, 0}, {0, 1}}, {{1, 1}, {0, 1}, {1, 0}}};
+    for (int64_t i = 0; i < ncopies; ++i) {
+        const int u = uid[i], l = (int)(i % nr), c = (int)(i / nr), Y = c % nx, X = (c / nx) % nx, sd = c / (nx * nx);
+        int32_t *row = &col[(size_t)u * kWidth];
+        for (int q = 0; q < 12; ++q) {
+            int dx, dy, w, dr, corner;
+            wedge_around(q, dx, dy, w, dr, corner);
+            const int xc = X + dx, yc = Y + dy, rc = l + dr;
+            if (xc < 0 || xc >= nc || yc < 0 || yc >= nc || rc < 0 || rc >= ncr) continue;
+            TNG_REQUIRE(xc + WN[w][corner][0] == X && yc + WN[w][corner][1] == Y, "coarse PCG: wedge table");
+            for (int k = 0; k < 6; ++k) {
+                const int32_t v = uid[m.lin(sd, xc + WN[w][k % 3][0], yc + WN[w][k % 3][1], rc + k / 3)];
+                int s = 0;
+                while (s < kWidth && row[s] >= 0 && row[s] != v) ++s;
+                TNG_REQUIRE(s < kWidth, "coarse PCG: a node with more neighbours than a row holds");
+                row[s] = v;
+                slot[(size_t)i * kMaxSlots + 6 * q + k] = (uint8_t)s;
+            }
+        }
+    }
+    upload(d_uid, uid.data(), uid.size() * sizeof(int32_t));
+    upload(d_rep, rep.data(), rep.size() * sizeof(int32_t));
+    upload(d_copy_begin, begin.data(), begin.size() * sizeof(int32_t));
+    upload(d_copy_list, list.data(), list.size() * sizeof(int32_t));
+    upload(d_slot, slot.data(), slot.size());
+    upload(d_col, col.data(), col.size() * sizeof(int32_t));
+    d_A.alloc((size_t)nu * 9 * kWidth * sizeof(double));
+    // x, r, A p, two directions, two sets of partials, the state
+    const std::vector<double> zero(CS_N, 0.0);
+    d_vec.alloc(((size_t)5 * 3 * nu + 2 * kCpcgMaxParts) * sizeof(double));
+    upload(d_state, zero.data(), zero.size() * sizeof(double));
+}
+
+void CoarsePcg::build(tng_operator &A, hipStream_t s)
+{
+    const tng_domain &m = *A.mesh;
+    if (!d_uid.p) numbering(m);
+    if (!A.stored) epsdivdiv_local_matrices(A, d_local, s);
+    TNG_REQUIRE(!A.stored || A.lmat_dtype == TNG_F64, "coarse PCG: FP64 matrices required");
+    CpcgArgs a{};
+    a.lmat = A.stored ? A.d_lmat.as<double>() : d_local.as<double>();
+    a.rep = d_rep.as<int32_t>();
+    a.copy_begin = d_copy_begin.as<int32_t>();
+    a.copy_list = d_copy_list.as<int32_t>();
+    a.slot = d_slot.as<uint8_t>();
+    a.col = d_col.as<int32_t>();
+    a.coords = m.d_coords.as<double>();
+    a.sd_cmb = m.d_sd_cmb.as<uint8_t>();
+    a.sd_surf = m.d_sd_surf.as<uint8_t>();
+    a.A = d_A.as<double>();
+    a.nu = nu; a.nx = m.nx; a.nr = m.nr; a.bc_cmb = A.bc_cmb; a.bc_surf = A.bc_surf;
+    hipLaunchKernelGGL(cpcg_assemble_kernel, dim3((nu * 9 + 63) / 64), dim3(64), 0, s, a);
+    hipLaunchKernelGGL(cpcg_boundary_kernel, dim3((nu * kWidth + 63) / 64), dim3(64), 0, s, a);
+    TNG_HIP_CHECK(hipGetLastError());
+    ready = true;
+}
+
+void CoarsePcg::solve(tng_vector &e0, const tng_vector &r0, int max_it, double rtol, double atol, hipStream_t s)
+{
+    TNG_REQUIRE(ready, "coarse PCG: not built");
+    // the host looks for an early end this often; until then the launches of a
+    // finished solve return at once
+    constexpr int kCheckEvery = 25;
+    const int n = 3 * nu, gu = (n + 255) / 256, gm = (nu + kCpcgNodes - 1) / kCpcgNodes;
+    double *x = d_vec.as<double>(), *r = x + n, *ap = r + n, *p[2] = {ap + n, ap + 2 * n};
+    double *rparts = ap + 3 * n, *pparts = rparts + kCpcgMaxParts, *st = d_state.as<double>();
+    TNG_REQUIRE(gm <= kCpcgMaxParts && gu <= kCpcgMaxParts, "coarse PCG: too many blocks");
+    const int32_t *uid = d_uid.as<int32_t>(), *rep = d_rep.as<int32_t>();
+    auto begin = [&](auto tag) {
+        using T = decltype(tag);
+        hipLaunchKernelGGL(cpcg_begin_kernel<T>, dim3(gu), dim3(256), 0, s,
+                           Comp3<const T>{{(const T *)r0.comp(0), (const T *)r0.comp(1), (const T *)r0.comp(2)}}, rep, nu,
+                           x, r, p[0], rparts, st);
+    };
+    if (r0.dtype == TNG_F64) begin(double());
+    else begin(float());
+    for (int it = 1; it <= max_it; ++it) {
+        hipLaunchKernelGGL(cpcg_matrix_kernel, dim3(gm), dim3(256), 0, s, d_A.as<double>(), d_col.as<int32_t>(), nu, r,
+                           p[(it - 1) & 1], p[it & 1], ap, rparts, gu, pparts, st, it, rtol, atol);
+        hipLaunchKernelGGL(cpcg_update_kernel, dim3(gu), dim3(256), 0, s, n, x, r, p[it & 1], ap, pparts, gm, rparts, st,
+                           it, max_it);
+        if (it % kCheckEvery == 0 && it < max_it) {
+            double done = 0.0;
+            TNG_HIP_CHECK(hipMemcpyAsync(&done, st + CS_DONE, sizeof(double), hipMemcpyDeviceToHost, s));
+            TNG_HIP_CHECK(hipStreamSynchronize(s));
+            if (done != 0.0) break;
+        }
+    }
+    auto scatter = [&](auto tag) {
+        using T = decltype(tag);
+        hipLaunchKernelGGL(scatter_kernel<T>, dim3(blocks(ncopies)), dim3(256), 0, s, (T *)e0.comp(0), (T *)e0.comp(1),
+                           (T *)e0.comp(2), uid, ncopies, (const double *)x);
+    };
+    if (e0.dtype == TNG_F64) scatter(double());
+    else scatter(float());
+    TNG_HIP_CHECK(hipGetLastError());
+}
+
+long CoarsePcg::take_iterations(hipStream_t s)
+{
+    if (!d_state.p) return 0;
+    double total = 0.0;
+    const double zero = 0.0;
+    double *slot = d_state.as<double>() + CS_TOTAL;
+    TNG_HIP_CHECK(hipMemcpyAsync(&total, slot, sizeof(double), hipMemcpyDeviceToHost, s));
+    TNG_HIP_CHECK(hipMemcpyAsync(slot, &zero, sizeof(double), hipMemcpyHostToDevice, s));
+    TNG_HIP_CHECK(hipStreamSynchronize(s));
+    return (long)total;
 }
 
 }  // namespace tng

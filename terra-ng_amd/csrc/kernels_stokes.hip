@@ -1272,7 +1272,7 @@ __global__ __launch_bounds__(256) void kmass_lumped_kernel(const T *k, const T *
 //   dst = 1/24 sum_t |det L_t| (2 W_own + W_a + W_b).
 // Bound by its loads (21 per component, all but the own three from cache).
 // Level 6, one component, FP64: 1690 us with all six points of the twelve
-// wedges evaluated per node, kMassTime now.
+// wedges evaluated per node, 50 us now.
 template <typename T>
 __global__ __launch_bounds__(256) void vector_mass_kernel(const Comp3<const T> src, const Comp3<T> dst, const double *radii,
                                                           const T *latgeom, int nsd, int nx, int nr, int ncomp,

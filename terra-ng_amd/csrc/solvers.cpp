@@ -204,6 +204,10 @@ void Multigrid::coarse_solve(tng_vector &e0, const tng_vector &r0, bool x_zero)
         coarse_iterations += 1;
         return;
     }
+    if (x_zero && pcg.ready) {
+        pcg.solve(e0, r0, coarse_max_it, coarse_rtol, coarse_atol, stream_of(e0));
+        return;
+    }
     // The coarsest solve runs in FP64 whatever the precision of the levels.
     tng_vector &x = e0.dtype == TNG_F64 ? e0 : *cg_x;
     const tng_vector *b = &r0;
@@ -449,6 +453,10 @@ void StokesSolver::viscosity_updated()
     if (mg.use_direct)
         mg.direct.build(*mg.coarse_op, *mg.cg_tmp[0], *mg.cg_tmp[1], params.viscous_pc_dtype != TNG_F64,
                         stream_of(*mg.cg_tmp[0]));
+    // PCG on a small coarsest level without the rotation penalty runs on the
+    // assembled operator: two launches per iteration instead of seven
+    else if (CoarsePcg::accepts(*mg.coarse_op))
+        mg.pcg.build(*mg.coarse_op, vel->ctx->stream);
     // k_pm = 1 / eta at the pressure level; lumped diagonal, inverted (DiagonalSolver)
     assign(*k_pm, *eta[nl - 2]);
     launch_invert(*k_pm, stream_of(*k_pm));
@@ -1041,10 +1049,11 @@ void StokesSolver::solve(SVec &x, const SVec &b, tng_solve_report &rep)
     rep.history = hist;
     rep.history_capacity = cap;
     mg.coarse_iterations = 0;
+    mg.pcg.take_iterations(vel->ctx->stream);
     if (params.rotation_correction && rc_dirty) rotation_setup();
     if (params.krylov_orthogonalization == 1) fgmres_cgs2(x, b, rep);
     else fgmres(x, b, rep);
-    rep.coarse_iterations = mg.coarse_iterations;
+    rep.coarse_iterations = mg.coarse_iterations + mg.pcg.take_iterations(vel->ctx->stream);
     // subtract the pressure mean over the unique pressure nodes (stokes_solver.hpp:680-689)
     const double avg = dot(*x.p, *ones_p) / (double)num_dofs_pressure;
     lincomb(*x.p, {1.0}, {x.p}, -avg);

@@ -52,6 +52,8 @@ struct Multigrid {
     // direct coarse solve (coarse_solver = 1), built with the viscosity
     bool use_direct = false;
     CoarseDirect direct;
+    // PCG on the assembled operator, built with the viscosity where it is accepted
+    CoarsePcg pcg;
 
     void solve(tng_vector &x, const tng_vector &b, bool x_zero = false);
     void recurse(int level, tng_vector &x, const tng_vector &b, bool x_zero);

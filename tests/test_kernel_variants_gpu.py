@@ -64,3 +64,22 @@ def test_mass_matches_oracle(L, Lr, ls, rs, gpu_ctx):
         out = vec(dom, u, dtype)
         tng.VectorMass(dom).apply(vec(dom, u, dtype), out)
         assert rel_err(out.download(), O.vector_mass(om, u)) < tol
+
+
+# the assembled coarse PCG: run to convergence it is the direct solve (relative residual 1e-13 times a condition
+# number of some 1e4), whatever the boundary rows, split diamonds, or Galerkin / re-discretised coarsest operator
+@pytest.mark.parametrize("bcs", [(D, D), (F, D), (D, F), (tng.NEUMANN, D)])
+@pytest.mark.parametrize("gca,sdr,dtype", [(0, 0, tng.F64), (1, 1, tng.F64), (1, 0, tng.F32)])
+def test_assembled_coarse_pcg_solves_the_coarse_system(bcs, gca, sdr, dtype, gpu_ctx):
+    om = O.Mesh(3, 3, 0.55, 1.0, sdr, 0)
+    eta, b = np.exp(0.5 * field(om, 1, 11)), field(om, 3, 12)
+    out = []
+    for kw in (dict(coarse_solver=1), dict(coarse_solver=0, coarse_max_iterations=4000, coarse_relative_tolerance=1e-13)):
+        S = tng.StokesSolver(2, 3, 0.55, 1.0, bcs, tng.StokesParams.defaults(gca=gca, viscous_pc_dtype=dtype, **kw),
+                             lateral_sdr=sdr)
+        dv = S.domain_velocity
+        S.set_viscosity(vec(dv, eta))
+        x = tng.VectorQ1Vec(dv)
+        S.precondition_velocity(x, vec(dv, b))
+        out.append(x.download())
+    assert rel_err(out[1], out[0]) < (1e-8 if dtype == tng.F64 else 1e-6)
