@@ -56,6 +56,9 @@ template <typename T> struct ApplyArgs {
     T *dst0, *dst1, *dst2;
     const T *k;
     const T *radii;     // (nsd, nr)
+    // the same in FP64: a layer's thickness is the difference of two radii, of
+    // which FP32 values keep few digits (128 layers: 1e-5 relative)
+    const double *radii64;
     const T *latgeom;   // (nsd, nc, nc, 2, 10)
     const T *coords;    // (nsd, nx, nx, 3) unit vectors (the radial normal)
     const T *btab;      // (nsd, nx, nx, 2, 3) boundary rows
@@ -451,11 +454,11 @@ __global__ __launch_bounds__(NW * 64) void epsdivdiv_apply_kernel(const ApplyArg
     #pragma unroll
         for (int p = 0; p < K; ++p) {
             const int l = lvl0 + p;
-            const T r0 = a.radii[(int64_t)sd * nr + l], r1 = a.radii[(int64_t)sd * nr + l + 1];
-            const T rmid = T(0.5) * (r0 + r1), h = T(0.5) * (r1 - r0);
-            const T hs = T(0.5) / rmid, tt = T(1) / (T(6) * h);
-            qq[p] = tt / hs;
-            cv[p] = lane_has ? hs * hs * rmid * rmid * h * T(1.0 / 6.0) : T(0);
+            const double r0 = a.radii64[(int64_t)sd * nr + l], r1 = a.radii64[(int64_t)sd * nr + l + 1];
+            const double rmid = 0.5 * (r0 + r1), h = 0.5 * (r1 - r0);
+            const double hs = 0.5 / rmid, tt = 1.0 / (6.0 * h);
+            qq[p] = (T)(tt / hs);
+            cv[p] = lane_has ? (T)(hs * hs * rmid * rmid * h * (1.0 / 6.0)) : T(0);
         }
 
         auto colbase = [&](int Xq, int Yq) -> int64_t {
@@ -931,7 +934,8 @@ __global__ __launch_bounds__(NW * 64) void epsdivdiv_apply_kernel(const ApplyArg
 template <typename T> struct DiagArgs {
     const T *src0, *src1, *src2;
     T *dst0, *dst1, *dst2;
-    const T *k, *radii, *latgeom, *coords;
+    const T *k, *latgeom, *coords;
+    const double *radii;  // FP64 in either precision, see ApplyArgs
     T *btab;
     const uint8_t *sd_cmb, *sd_surf;
     int nsd, nx, nr, ncells, bc_cmb, bc_surf, add, mode;
@@ -1029,8 +1033,8 @@ template <typename T> __global__ void epsdivdiv_diag_kernel(const DiagArgs<T> a)
                 const T l1 = kc == 0 ? T(-0.5) : (kc == 1 ? T(0) : T(0.5));
                 for (int rc = l - 1; rc <= l; ++rc) {
                     if (rc < 0 || rc >= a.ncells) continue;
-                    const T r0 = a.radii[(int64_t)sd * nr + rc], r1 = a.radii[(int64_t)sd * nr + rc + 1];
-                    const T rmid = T(0.5) * (r0 + r1), h = T(0.5) * (r1 - r0);
+                    const double r0 = a.radii[(int64_t)sd * nr + rc], r1 = a.radii[(int64_t)sd * nr + rc + 1];
+                    const T rmid = (T)(0.5 * (r0 + r1)), h = (T)(0.5 * (r1 - r0));
                     const T s = T(1) / rmid;
                     const T dz = (rc == l) ? T(-1.0 / 6.0) : T(1.0 / 6.0);
                     T gv[3];
@@ -1385,7 +1389,7 @@ template <typename T> void run_diag_kernel(tng_operator &op, const tng_vector *s
         a.dst0 = (T *)dst->comp(0); a.dst1 = (T *)dst->comp(1); a.dst2 = (T *)dst->comp(2);
     }
     a.k = (const T *)op.k->comp(0);
-    a.radii = mp.radii; a.latgeom = mp.latgeom; a.coords = mp.coords;
+    a.radii = m.d_radii.as<double>(); a.latgeom = mp.latgeom; a.coords = mp.coords;
     a.btab = op.d_btab.as<T>();
     a.sd_cmb = m.d_sd_cmb.as<uint8_t>(); a.sd_surf = m.d_sd_surf.as<uint8_t>();
     a.nsd = m.nsd; a.nx = m.nx; a.nr = m.nr; a.ncells = m.nr - 1;
@@ -1458,6 +1462,7 @@ ApplyArgs<T> apply_args(const tng_operator &op, const tng_vector &src, tng_vecto
     a.dst0 = (T *)dst.comp(0); a.dst1 = (T *)dst.comp(1); a.dst2 = (T *)dst.comp(2);
     a.k = (const T *)op.k->comp(0);
     a.radii = mp.radii; a.latgeom = mp.latgeom; a.coords = mp.coords;
+    a.radii64 = m.d_radii.as<double>();
     a.btab = op.d_btab.as<T>();
     a.pen = pen ? op.d_penalty_b.as<double>() : nullptr;
     a.sd_cmb = m.d_sd_cmb.as<uint8_t>(); a.sd_surf = m.d_sd_surf.as<uint8_t>();
