@@ -1481,6 +1481,17 @@ void apply_impl(tng_operator &op, const tng_vector &src, tng_vector &dst, hipStr
     const bool add = op.apply_mode == TNG_ADD;
     hipEvent_t *ev = ctx.profiling && !ws ? ctx.prof_next_set() : nullptr;
     if (ev) TNG_HIP_CHECK(hipEventRecord(ev[0], s));
+    if (fan_applies(op)) {
+        // 4 to 32 radial layers without penalty: one launch, halo sum included
+        if (!op.btab_valid) epsdivdiv_update_boundary_table(op, s);
+        if (ev) TNG_HIP_CHECK(hipEventRecord(ev[1], s));
+        fan_apply(op, src, dst, s);
+        if (ev) {
+            TNG_HIP_CHECK(hipEventRecord(ev[2], s));
+            TNG_HIP_CHECK(hipEventRecord(ev[3], s));
+        }
+        return;
+    }
     double *partials = ws ? ws : m.ctx->red_partials.as<double>();
     auto penalty_moment = [&]() { tng::penalty_moment<T>(op, src, s, partials); };
     if (op.stored) {
@@ -1543,6 +1554,18 @@ bool apply_cheb_impl(tng_operator &op, const tng_vector &x, tng_vector &ax, tng_
     if (op.stored || op.diagonal || op.apply_mode != TNG_REPLACE || op.comm_mode != TNG_COMMUNICATE_ADDITIVELY ||
         m.rad_sdr != 0)
         return false;
+    if (fan_applies(op)) {
+        hipEvent_t *ev = m.ctx->profiling ? m.ctx->prof_next_set() : nullptr;
+        if (ev) TNG_HIP_CHECK(hipEventRecord(ev[0], s));
+        if (!op.btab_valid) epsdivdiv_update_boundary_table(op, s);
+        if (ev) TNG_HIP_CHECK(hipEventRecord(ev[1], s));
+        fan_apply_cheb(op, x, x_out, d, b, invd, az, ad, read_d, s);
+        if (ev) {
+            TNG_HIP_CHECK(hipEventRecord(ev[2], s));
+            TNG_HIP_CHECK(hipEventRecord(ev[3], s));
+        }
+        return true;
+    }
     const ApplyShape sh = apply_shape(m.nr - 1, m.ctx->tuning, true);
     if (!(sh.R == 64 && sh.K == 1 && sh.NW == 8 && sh.RG <= 2 && sh.S == 1)) return false;
     tng_context &ctx = *m.ctx;

@@ -205,6 +205,33 @@ void mesh_build(tng_domain &m, int lat_level, int rad_level, double r_min, doubl
         lat_groups.back().push_back(keys[i].second);
         lat_id[keys[i].second] = (int64_t)lat_groups.size() - 1;
     }
+    // task table of the fan apply: groups of copies in the order of their first
+    // column, none across two blocks
+    const int ncr = nr - 1;
+    if (rad_sdr == 0 && ncr >= 4 && ncr <= 32) {
+        const int cap = (ncr == 32 ? 512 : 256) / (2 * ncr);  // as kFanCap
+        std::vector<int64_t> order;
+        for (size_t g = 0; g < lat_groups.size(); ++g) order.push_back((int64_t)g);
+        std::sort(order.begin(), order.end(),
+                  [&](int64_t a, int64_t b) { return lat_groups[a].front() < lat_groups[b].front(); });
+        for (const int64_t g : order) {
+            const auto &cols = lat_groups[g];  // ascending (sorted keys carry the column)
+            TNG_REQUIRE((int)cols.size() <= cap, "more copies of a lateral node than a block holds");
+            const int used = (int)(m.fan_col.size() % cap);
+            if (used + (int)cols.size() > cap) {
+                m.fan_col.resize(m.fan_col.size() + cap - used, -1);
+                m.fan_grp.resize(m.fan_col.size(), 1 << 8);
+            }
+            const int first = (int)(m.fan_col.size() % cap);
+            for (const int64_t c : cols) {
+                m.fan_col.push_back((int32_t)c);
+                m.fan_grp.push_back(first | (int)cols.size() << 8);
+            }
+        }
+        m.fan_blocks = (int)((m.fan_col.size() + cap - 1) / cap);
+        m.fan_col.resize((size_t)m.fan_blocks * cap, -1);
+        m.fan_grp.resize((size_t)m.fan_blocks * cap, 1 << 8);
+    }
     // ownership: MIN global subdomain id among the copies (grid/bit_masks.hpp:29-85;
     // SubdomainInfo::global_id, spherical_shell.hpp:696-722)
     auto gid = [&](int sd) {
@@ -308,6 +335,10 @@ void mesh_upload(tng_domain &m)
     up(m.d_bmask, m.bmask.data(), m.bmask.size());
     up(m.d_sd_cmb, m.sd_has_cmb.data(), m.sd_has_cmb.size());
     up(m.d_sd_surf, m.sd_has_surf.data(), m.sd_has_surf.size());
+    if (m.fan_blocks > 0) {
+        up(m.d_fan_col, m.fan_col.data(), m.fan_col.size() * sizeof(int32_t));
+        up(m.d_fan_grp, m.fan_grp.data(), m.fan_grp.size() * sizeof(int32_t));
+    }
     std::vector<float> cf(m.coords.begin(), m.coords.end()), rf(m.radii.begin(), m.radii.end());
     up(m.d_coords_f, cf.data(), cf.size() * sizeof(float));
     up(m.d_radii_f, rf.data(), rf.size() * sizeof(float));

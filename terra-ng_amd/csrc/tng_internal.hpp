@@ -167,6 +167,12 @@ struct tng_domain {
     int halo_maxc = 0;
     int64_t halo_n = 0;
     tng::DevBuf d_halo_idx;
+    // task table of the fan apply (kernels_fan.hip): blocks of 8 or more
+    // lateral columns, the copies of a shared lateral node in one block; absent
+    // (fan_blocks = 0) where that kernel does not apply
+    int fan_blocks = 0;
+    std::vector<int32_t> fan_col, fan_grp;
+    tng::DevBuf d_fan_col, d_fan_grp;
     // Gram matrix of the rotation fields e_j x x over OWNED nodes (inverse).
     double rot_gram_inv[9] = {0};
 
@@ -305,6 +311,12 @@ void epsdivdiv_apply_noalloc(tng_operator &op, const tng_vector &src, tng_vector
 bool epsdivdiv_apply_cheb(tng_operator &op, const tng_vector &x, tng_vector &ax, tng_vector &x_out, tng_vector &d,
                           const tng_vector &b, const tng_vector &invd, double az, double ad, bool read_d,
                           hipStream_t s);
+// The same for 4 to 32 radial layers in one launch (kernels_fan.hip): apply,
+// halo sum and, in the second, the sub-step.
+bool fan_applies(const tng_operator &op);
+void fan_apply(tng_operator &op, const tng_vector &src, tng_vector &dst, hipStream_t s);
+void fan_apply_cheb(tng_operator &op, const tng_vector &x, tng_vector &x_out, tng_vector &d, const tng_vector &b,
+                    const tng_vector &invd, double az, double ad, bool read_d, hipStream_t s);
 // XDMF field layout: pack (device layout -> file layout, out_bytes 4 or 8)
 // and unpack; checkpoint read of one field (io/xdmf.hpp:1199-1441).
 void xdmf_pack(const tng_vector &v, void *dst_device, int out_bytes, hipStream_t s);

@@ -83,3 +83,56 @@ def test_assembled_coarse_pcg_solves_the_coarse_system(bcs, gca, sdr, dtype, gpu
         S.precondition_velocity(x, vec(dv, b))
         out.append(x.download())
     assert rel_err(out[1], out[0]) < (1e-8 if dtype == tng.F64 else 1e-6)
+
+
+# the fan kernel: every lane-group size (4 to 32 layers; 32 in FP32 only, FP64 takes the sweep there), shared nodes of
+# two to five copies inside and across diamonds, every boundary mix, Add mode and skipped communication
+@pytest.mark.parametrize("L,Lr,ls", [(2, 2, 1), (3, 3, 2), (3, 4, 1), (4, 5, 0), (1, 3, 0), (5, 2, 2)])
+@pytest.mark.parametrize("bcs", [(D, D), (F, D), (D, F), (tng.NEUMANN, F), (tng.NEUMANN, tng.NEUMANN)])
+def test_fan_apply_matches_oracle(L, Lr, ls, bcs, gpu_ctx):
+    dom = tng.DistributedDomain.create_uniform(L, Lr, 0.55, 1.0, ls, 0)
+    om = O.Mesh(L, Lr, 0.55, 1.0, ls, 0)
+    k, u, base = np.exp(0.5 * field(om, 1, 21)), field(om, 3, 22), field(om, 3, 23)
+    # FP32: inputs and tables rounded to 6e-8, gradients over thin cells lose about their aspect ratio
+    for dtype, tol in ((tng.F64, 1e-12), (tng.F32, 1e-5)):
+        kv, uv = vec(dom, k, dtype), vec(dom, u, dtype)
+        op = tng.EpsilonDivDivKerngen(dom, kv, bcs)
+        out = vec(dom, base, dtype)
+        op.apply(uv, out)
+        assert rel_err(out.download(), om.epsdivdiv(k, u, *bcs)) < tol
+        for mode in ((tng.ADD, tng.SKIP_COMMUNICATION), (tng.ADD, tng.COMMUNICATE_ADDITIVELY),
+                     (tng.REPLACE, tng.SKIP_COMMUNICATION)):
+            op.set_operator_apply_and_communication_modes(*mode)
+            out = vec(dom, base, dtype)
+            op.apply(uv, out)
+            ref = om.epsdivdiv(k, u, *bcs, apply_mode=mode[0], comm=mode[1], dst=base)
+            assert rel_err(out.download(), ref) < tol
+
+
+# copies that differ (a vector that no exchange has made consistent): each copy's cells read their own subdomain's values
+def test_fan_apply_reads_each_subdomains_own_copies(gpu_ctx):
+    dom, om = tng.DistributedDomain.create_uniform(3, 3, 0.55, 1.0, 1, 0), O.Mesh(3, 3, 0.55, 1.0, 1, 0)
+    k = np.exp(0.5 * field(om, 1, 24))
+    u = np.random.default_rng(25).uniform(-1, 1, (3,) + om.shape)
+    for bcs in ((D, F), (F, D)):
+        out = vec(dom, u)
+        tng.EpsilonDivDivKerngen(dom, vec(dom, k), bcs).apply(vec(dom, u), out)
+        assert rel_err(out.download(), om.epsdivdiv(k, u, *bcs)) < 1e-12
+
+
+@pytest.mark.parametrize("dtype", [tng.F64, tng.F32])
+@pytest.mark.parametrize("bcs,sdr", [((D, D), 0), ((D, F), 1)])
+def test_fan_chebyshev_has_the_bits_of_the_separate_kernels(dtype, bcs, sdr, gpu_ctx):
+    om = O.Mesh(5, 5, 0.55, 1.0, sdr, 0)
+    eta, b = np.exp(0.5 * field(om, 1, 26)), field(om, 3, 27)
+    out = []
+    for fuse in (0, 1):
+        with tng.default_context().tuning(cheb_fuse=fuse):
+            S = tng.StokesSolver(2, 5, 0.55, 1.0, bcs, tng.StokesParams.defaults(
+                viscous_pc_dtype=dtype, viscous_pc_chebyshev_order=3, coarse_solver=1), lateral_sdr=sdr)
+        S.set_viscosity(vec(S.domain_velocity, eta))
+        x = tng.VectorQ1Vec(S.domain_velocity)
+        for _ in range(2):  # from zero, then from a start vector
+            S.precondition_velocity(x, vec(S.domain_velocity, b))
+        out.append(x.download())
+    assert np.array_equal(out[0], out[1])
