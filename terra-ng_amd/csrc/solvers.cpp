@@ -230,9 +230,8 @@ void Multigrid::recurse(int level, tng_vector &x, const tng_vector &b, bool x_ze
     Level &L = levels[level];
     pre[level].solve(*L.A, x, b, x_zero);
     apply(*L.A, x, *L.tmp);
-    lincomb(*L.tmp, {1.0, -1.0}, {&b, L.tmp});
     Level &C = levels[level - 1];
-    apply(*L.R, *L.tmp, *C.r);
+    restrict_residual(*L.R, *L.tmp, b, *C.r, stream_of(x));
     assign(*C.e, 0.0);
     recurse(level - 1, *C.e, *C.r, true);
     apply(*L.P, *C.e, x);  // Add mode

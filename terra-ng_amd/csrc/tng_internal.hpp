@@ -325,6 +325,8 @@ void xdmf_checkpoint_read(const std::string &dir, const std::string &label, int 
 void launch_halo_cheb(const tng_domain &m, const tng_vector &ax, const tng_vector &b, const tng_vector &invd,
                       tng_vector &d, const tng_vector &x, tng_vector &x_out, double az, double ad, bool read_d,
                       hipStream_t s);
+// dst = R (b - ax), the restriction with its additive exchange
+void restrict_residual(tng_operator &R, const tng_vector &ax, const tng_vector &b, tng_vector &dst, hipStream_t s);
 void stokes_block_apply(tng_operator &op, const tng_vector &src, tng_vector &dst, hipStream_t s);
 
 // BLAS-1 and reductions (kernels_vec.hip)
