@@ -344,6 +344,43 @@ __device__ __forceinline__ void cheb_update(const ApplyArgs<T> &a, int64_t i, co
     }
 }
 
+// The same for a run of two consecutive levels, moved as pairs (a column starts
+// at any multiple of one value).  b, invd and d are read and d and x written
+// once per sub-step of a level that no cache holds: they pass by the caches, so
+// that the columns of x and k stay for the neighbouring strips.
+template <typename T> using RunPair = T __attribute__((ext_vector_type(2), aligned(sizeof(T))));
+
+template <typename T>
+__device__ __forceinline__ void cheb_update_pair(const ApplyArgs<T> &a, int64_t i, const T (&val)[2][3])
+{
+#pragma clang fp contract(off)
+    const T *cb[3] = {a.cb0, a.cb1, a.cb2}, *ci[3] = {a.ci0, a.ci1, a.ci2}, *xs[3] = {a.src0, a.src1, a.src2};
+    T *cd[3] = {a.cd0, a.cd1, a.cd2}, *cx[3] = {a.cx0, a.cx1, a.cx2};
+    RunPair<T> b[3], v[3], d[3], x[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        b[c] = __builtin_nontemporal_load((const RunPair<T> *)(cb[c] + i));
+        v[c] = __builtin_nontemporal_load((const RunPair<T> *)(ci[c] + i));
+        if (a.cread_d) d[c] = __builtin_nontemporal_load((const RunPair<T> *)(cd[c] + i));
+        x[c] = *(const RunPair<T> *)(xs[c] + i);
+    }
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        RunPair<T> dn, xn;
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            const T r = b[c][p] - val[p][c];
+            const T z = r * v[c][p];
+            T t = a.caz * z;
+            if (a.cread_d) t = fma(a.cad, d[c][p], t);
+            dn[p] = t;
+            xn[p] = x[c][p] + t;
+        }
+        __builtin_nontemporal_store(dn, (RunPair<T> *)(cd[c] + i));
+        __builtin_nontemporal_store(xn, (RunPair<T> *)(cx[c] + i));
+    }
+}
+
 template <typename T, int R, int K, int NW, int RG, int BCM, bool FUSE, bool SPLIT>
 __global__ __launch_bounds__(NW * 64) void epsdivdiv_apply_kernel(const ApplyArgs<T> a)
 {
@@ -358,12 +395,15 @@ __global__ __launch_bounds__(NW * 64) void epsdivdiv_apply_kernel(const ApplyArg
     constexpr int VX = NW / RG * VPW;
     constexpr int NV = VX * RG;
     constexpr int KL = K + 1;
+    // scalar geometry and a sweep unrolled by two, where the registers allow it
+    constexpr bool two_steps = K == 1 || (K == 2 && sizeof(T) == 4);
     // left-corner contributions of every cell for rows yc (corner 00) and
     // yc+1 (corner 01), lateral part L and radial part C apart, per virtual
     // column, double-buffered by step parity (one cell per lane; more cells
-    // per lane use one buffer and a second barrier); the last cell's own L
-    // and C of a lower chunk's top lane (before the lateral exchange)
-    constexpr int NB = K == 1 ? 2 : 1;
+    // per lane: four use one buffer and a second barrier); the last cell's own L
+    // and C of a lower chunk's top lane (before the lateral exchange).  Two
+    // cells per lane, L7 FP32 V-cycle: 8.63 ms with one buffer, 8.53 with two
+    constexpr int NB = K <= 2 ? 2 : 1;
     __shared__ T xch[NB][NV][2][2][K][3][R];
     __shared__ T xtop[NB][RG > 1 ? NV : 1][2][3];
 
@@ -578,7 +618,7 @@ __global__ __launch_bounds__(NW * 64) void epsdivdiv_apply_kernel(const ApplyArg
             // new row to arrive (more cells per lane run out of scalar registers
             // and take it from the record instead)
             T sg[20];
-            if constexpr (R == 64 && K == 1 && TNG_APPLY_SMEM_GEOM) {
+            if constexpr (R == 64 && two_steps && TNG_APPLY_SMEM_GEOM) {
                 using CT = const T __attribute__((address_space(4)));
                 const int xcc = min(max(xc, 0), nc - 1), ycc = min(max(yc, 0), nc - 1);
                 const int gi = __builtin_amdgcn_readfirstlane(((sd * nc + xcc) * nc + ycc) * 20);
@@ -625,7 +665,7 @@ __global__ __launch_bounds__(NW * 64) void epsdivdiv_apply_kernel(const ApplyArg
             const bool cell_ok = xc >= 0 && xc < nc && yc >= 0 && yc < nc;
             {
                 T g0[10], g1[10];
-                if constexpr (R == 64 && K == 1 && TNG_APPLY_SMEM_GEOM) {
+                if constexpr (R == 64 && two_steps && TNG_APPLY_SMEM_GEOM) {
     #pragma unroll
                     for (int i = 0; i < 10; ++i) {
                         g0[i] = sg[i];
@@ -767,6 +807,9 @@ __global__ __launch_bounds__(NW * 64) void epsdivdiv_apply_kernel(const ApplyArg
                     pbn[1] = fma(pb[2], cc[0], -(pb[0] * cc[2]));
                     pbn[2] = fma(pb[0], cc[1], -(pb[1] * cc[0]));
                 }
+                // two cells per lane: the lane's run of levels is stored at the end
+                constexpr bool run = K == 2 && two_steps;
+                T runv[2][3];
     #pragma unroll
                 for (int p = 0; p < KL; ++p) {
                     if (p == K && !(ovf_lane && top_chunk)) continue;
@@ -857,6 +900,13 @@ __global__ __launch_bounds__(NW * 64) void epsdivdiv_apply_kernel(const ApplyArg
                         val[1] += a.dst1[base + l];
                         val[2] += a.dst2[base + l];
                     }
+                    if constexpr (run) {
+                        if (p < K) {
+    #pragma unroll
+                            for (int c = 0; c < 3; ++c) runv[p < 2 ? p : 0][c] = val[c];
+                            continue;
+                        }
+                    }
                     if constexpr (FUSE) {
                         // columns off the subdomain's lateral edges are not shared
                         // (every subdomain spans the whole shell radially here)
@@ -886,6 +936,19 @@ __global__ __launch_bounds__(NW * 64) void epsdivdiv_apply_kernel(const ApplyArg
                     a.dst1[base + l] = val[1];
                     a.dst2[base + l] = val[2];
                 }
+                if constexpr (run) {
+                    const int64_t i = base + c0 + rl * K;
+                    if (FUSE && fuse_here) {
+                        cheb_update_pair<T>(a, i, runv);
+                    } else {
+                        T *ds[3] = {a.dst0, a.dst1, a.dst2};
+    #pragma unroll
+                        for (int c = 0; c < 3; ++c) {
+                            const RunPair<T> v = {runv[0][c], runv[1][c]};
+                            *(RunPair<T> *)(ds[c] + i) = v;
+                        }
+                    }
+                }
             }
     #pragma unroll
             for (int i = 0; i < K; ++i)
@@ -896,7 +959,7 @@ __global__ __launch_bounds__(NW * 64) void epsdivdiv_apply_kernel(const ApplyArg
         const int nsteps = Yend - (Y0 - 1);
         NodeCol<T, K> C0, C1;
         T rec2 = T(0);
-        if constexpr (R == 64 && K == 1) {
+        if constexpr (R == 64 && two_steps) {
             // two steps per iteration with alternating roles (no register copies)
             for (int step = 0; step < nsteps; step += 2) {
                 do_step(step, B0, B1, C0, C1, aLA, aCA, aLB, aCB, rec, rec2);
@@ -1270,11 +1333,24 @@ struct ApplyShape {
     int R, K, RG, NW, S;
 };
 
-ApplyShape apply_shape(int ncells, const tng_tuning &tu, bool fused = false)
+ApplyShape apply_shape(int ncells, const tng_tuning &tu, bool fused = false, bool f32 = false)
 {
     ApplyShape sh{64, 1, 1, 8, 1};
     const int chunks = tu.apply_radial_chunks;
     const bool split = tu.apply_radial_split != 0;
+    if (f32 && ncells == 128 && (fused ? chunks != 1 : chunks == 0 && split)) {
+        // FP32 is bound by vector instructions (a scalar FP32 operation costs
+        // what an FP64 one does).  Two cells per lane issue a quarter fewer of
+        // them than radial chunks or parts of 64 cells: strips of eight columns
+        // overlap by one (by one in four with two chunks), column records, rows of
+        // the exchange and boundary terms serve two cells, and a lane moves its
+        // levels as pairs.  10 x 129 x 129 columns: apply 312 us plus 15 us for
+        // the levels between parts -> 240 us; fused Chebyshev sub-step 536 us
+        // (two chunks) -> 486 us.  FP64 takes 64 cells per lane set: two cells
+        // of it exceed the 256 registers that two waves per SIMD leave.
+        sh.K = 2;
+        return sh;
+    }
     if (ncells >= 128 && chunks == 0 && split && !fused) {
         // radial parts of 64 cells swept like separate subdomains (eight
         // one-column waves per workgroup, seven new columns each), their
@@ -1302,12 +1378,12 @@ template <typename T, bool FUSE = false> void launch_apply(ApplyArgs<T> a, hipSt
     // shapes: up to 64 radial cells one cell per lane (R lanes per column);
     // more as radial parts of 64 cells, or (128 and 256 cells) radial chunks
     // of one wave each or K cells per lane
-    const ApplyShape sh = apply_shape(a.ncells, tu, FUSE);
+    const ApplyShape sh = apply_shape(a.ncells, tu, FUSE, sizeof(T) == 4);
     const int R = sh.R, K = sh.K, RG = sh.RG, NW = sh.NW;
     TNG_REQUIRE(K <= 4, "more than 256 radial layers per subdomain need the radial parts");
     a.rsplit = sh.S;
     TNG_REQUIRE(sh.S == 1 || (R == 64 && K == 1 && !FUSE && a.iface), "radial parts need the one-column kernels");
-    TNG_REQUIRE(!FUSE || (R == 64 && K == 1 && NW == 8 && RG <= 2),
+    TNG_REQUIRE(!FUSE || (R == 64 && K <= 2 && NW == 8 && RG <= 2),
                 "the fused Chebyshev step needs the one-column kernels with at most 128 radial layers");
     const int VX = NW / RG * (64 / R);
     // R = 64: strips over the columns of all subdomains in a row; otherwise
@@ -1340,11 +1416,13 @@ template <typename T, bool FUSE = false> void launch_apply(ApplyArgs<T> a, hipSt
             }
         }
     } else if (RG == 2) {
-        switch (bcm) {
-        case 0: launch_apply_rk<T, 64, 1, 8, 2, 0, FUSE>(a, lg, s, tu); break;
-        case 1: launch_apply_rk<T, 64, 1, 8, 2, 1, FUSE>(a, lg, s, tu); break;
-        case 2: launch_apply_rk<T, 64, 1, 8, 2, 2, FUSE>(a, lg, s, tu); break;
-        default: launch_apply_rk<T, 64, 1, 8, 2, 3, FUSE>(a, lg, s, tu); break;
+        if constexpr (!FUSE || sizeof(T) == 8) {  // the fused step in FP32 takes two cells per lane
+            switch (bcm) {
+            case 0: launch_apply_rk<T, 64, 1, 8, 2, 0, FUSE>(a, lg, s, tu); break;
+            case 1: launch_apply_rk<T, 64, 1, 8, 2, 1, FUSE>(a, lg, s, tu); break;
+            case 2: launch_apply_rk<T, 64, 1, 8, 2, 2, FUSE>(a, lg, s, tu); break;
+            default: launch_apply_rk<T, 64, 1, 8, 2, 3, FUSE>(a, lg, s, tu); break;
+            }
         }
     } else if (K == 1 && R == 64 && NW == 8) {
         switch (bcm) {
@@ -1352,6 +1430,15 @@ template <typename T, bool FUSE = false> void launch_apply(ApplyArgs<T> a, hipSt
         case 1: launch_apply_rk<T, 64, 1, 8, 1, 1, FUSE>(a, lg, s, tu); break;
         case 2: launch_apply_rk<T, 64, 1, 8, 1, 2, FUSE>(a, lg, s, tu); break;
         default: launch_apply_rk<T, 64, 1, 8, 1, 3, FUSE>(a, lg, s, tu); break;
+        }
+    } else if (sizeof(T) == 4 && K == 2 && NW == 8) {
+        if constexpr (sizeof(T) == 4) {
+            switch (bcm) {
+            case 0: launch_apply_rk<T, 64, 2, 8, 1, 0, FUSE>(a, lg, s, tu); break;
+            case 1: launch_apply_rk<T, 64, 2, 8, 1, 1, FUSE>(a, lg, s, tu); break;
+            case 2: launch_apply_rk<T, 64, 2, 8, 1, 2, FUSE>(a, lg, s, tu); break;
+            default: launch_apply_rk<T, 64, 2, 8, 1, 3, FUSE>(a, lg, s, tu); break;
+            }
         }
     } else if constexpr (FUSE) {
         // unreachable: rejected above
@@ -1510,10 +1597,12 @@ void apply_impl(tng_operator &op, const tng_vector &src, tng_vector &dst, hipStr
         // penalty: the per-block moments only; every apply workgroup combines them
         const bool pen = op.penalty_active;
         ApplyArgs<T> a = apply_args<T>(op, src, dst, false, add);
-        const ApplyShape sh = apply_shape(m.nr - 1, m.ctx->tuning);
-        if (sh.S > 1) {
-            // partial sums of the levels between radial parts
-            const size_t bytes = sizeof(T) * 6 * (sh.S - 1) * (size_t)m.nsd * m.nx * m.nx;
+        const ApplyShape sh = apply_shape(m.nr - 1, m.ctx->tuning, false, sizeof(T) == 4);
+        // partial sums of the levels between radial parts; the allocation-free
+        // apply takes the same meshes whether or not its type has parts
+        const int parts = ws ? apply_shape(m.nr - 1, m.ctx->tuning).S : sh.S;
+        if (parts > 1) {
+            const size_t bytes = sizeof(T) * 6 * (parts - 1) * (size_t)m.nsd * m.nx * m.nx;
             if (ws) {
                 TNG_REQUIRE(bytes <= kNoAllocScratchBytes - kNoAllocPenDoubles * sizeof(double),
                             "allocation-free apply: the partial sums between radial parts need " +
@@ -1566,8 +1655,8 @@ bool apply_cheb_impl(tng_operator &op, const tng_vector &x, tng_vector &ax, tng_
         }
         return true;
     }
-    const ApplyShape sh = apply_shape(m.nr - 1, m.ctx->tuning, true);
-    if (!(sh.R == 64 && sh.K == 1 && sh.NW == 8 && sh.RG <= 2 && sh.S == 1)) return false;
+    const ApplyShape sh = apply_shape(m.nr - 1, m.ctx->tuning, true, sizeof(T) == 4);
+    if (!(sh.R == 64 && sh.K <= 2 && sh.NW == 8 && sh.RG <= 2 && sh.S == 1)) return false;
     tng_context &ctx = *m.ctx;
     hipEvent_t *ev = ctx.profiling ? ctx.prof_next_set() : nullptr;
     if (ev) TNG_HIP_CHECK(hipEventRecord(ev[0], s));

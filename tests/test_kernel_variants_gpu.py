@@ -10,7 +10,7 @@ from conftest import consistent, rel_err
 
 pytestmark = pytest.mark.gpu
 
-D, F = tng.DIRICHLET, tng.FREESLIP
+D, F, N = tng.DIRICHLET, tng.FREESLIP, tng.NEUMANN
 
 
 def field(om, ncomp, seed, scale=1.0):
@@ -133,6 +133,42 @@ def test_fan_chebyshev_has_the_bits_of_the_separate_kernels(dtype, bcs, sdr, gpu
         S.set_viscosity(vec(S.domain_velocity, eta))
         x = tng.VectorQ1Vec(S.domain_velocity)
         for _ in range(2):  # from zero, then from a start vector
+            S.precondition_velocity(x, vec(S.domain_velocity, b))
+        out.append(x.download())
+    assert np.array_equal(out[0], out[1])
+
+
+# FP32 at 128 layers, two cells per lane: strips of eight columns within one subdomain and across several, every
+# boundary mix and the penalty, both apply modes, copies that differ
+@pytest.mark.parametrize("L,ls,rs", [(1, 0, 0), (2, 1, 0), (3, 0, 1)])
+@pytest.mark.parametrize("bcs", [(D, D), (F, F), (N, N), (F, D), (D, F), (N, F)])
+def test_fp32_pairs_of_cells_match_oracle(L, ls, rs, bcs, gpu_ctx):
+    dom, om = tng.DistributedDomain.create_uniform(L, 7 + rs, 0.55, 1.0, ls, rs), O.Mesh(L, 7 + rs, 0.55, 1.0, ls, rs)
+    k, base = np.exp(0.5 * field(om, 1, 28)), field(om, 3, 29)
+    u = np.random.default_rng(30).uniform(-1, 1, (3,) + om.shape)
+    op = tng.EpsilonDivDivKerngen(dom, vec(dom, k, tng.F32), bcs)
+    op.set_penalty_epsilon(1.0)
+    for mode in ((tng.REPLACE, tng.COMMUNICATE_ADDITIVELY), (tng.ADD, tng.SKIP_COMMUNICATION)):
+        op.set_operator_apply_and_communication_modes(*mode)
+        out = vec(dom, base, tng.F32)
+        op.apply(vec(dom, u, tng.F32), out)
+        ref = om.epsdivdiv(k, u, *bcs, path="fast", penalty_eps=1.0, apply_mode=mode[0], comm=mode[1], dst=base)
+        # inputs and tables rounded to 6e-8; differences over cells a hundred times flatter than wide lose two digits
+        assert rel_err(out.download(), ref) < 1e-5
+
+
+@pytest.mark.parametrize("bcs", [(D, D), (F, F), (D, F)])
+def test_fp32_pairs_fused_have_the_bits_of_the_separate_kernels(bcs, gpu_ctx):
+    om = O.Mesh(4, 7, 0.55, 1.0, 0, 0)
+    eta, b = np.exp(0.5 * field(om, 1, 31)), field(om, 3, 32)
+    out = []
+    for fuse in (0, 1):
+        with tng.default_context().tuning(cheb_fuse=fuse):
+            S = tng.StokesSolver(1, 4, 0.55, 1.0, bcs, tng.StokesParams.defaults(
+                viscous_pc_dtype=tng.F32, viscous_pc_chebyshev_order=3, coarse_solver=1), radial_extra_levels=3)
+        S.set_viscosity(vec(S.domain_velocity, eta))
+        x = tng.VectorQ1Vec(S.domain_velocity)
+        for _ in range(2):
             S.precondition_velocity(x, vec(S.domain_velocity, b))
         out.append(x.download())
     assert np.array_equal(out[0], out[1])
