@@ -172,3 +172,16 @@ def test_fp32_pairs_fused_have_the_bits_of_the_separate_kernels(bcs, gpu_ctx):
             S.precondition_velocity(x, vec(S.domain_velocity, b))
         out.append(x.download())
     assert np.array_equal(out[0], out[1])
+
+
+# the adjoint's wedge products: two layers (cells that meet at one node level), one and several rows per thread,
+# waves in one column (64 and 128 layers) and in several, radial subdomains without a boundary
+@pytest.mark.parametrize("L,Lr,ls,rs", [(1, 1, 0, 0), (2, 3, 1, 0), (2, 6, 0, 0), (1, 7, 0, 0), (3, 8, 0, 2), (5, 5, 0, 0),
+                                        (6, 6, 0, 0)])
+@pytest.mark.parametrize("bcs", [(N, N), (D, F), (F, D)])
+def test_adjoint_sweep_matches_oracle(L, Lr, ls, rs, bcs, gpu_ctx):
+    dom, om = tng.DistributedDomain.create_uniform(L, Lr, 0.55, 1.0, ls, rs), O.Mesh(L, Lr, 0.55, 1.0, ls, rs)
+    k, lam, u = np.exp(field(om, 1, 33)), field(om, 3, 34), field(om, 3, 35)
+    g = vec(dom, k)
+    tng.EpsilonDivDivKerngen(dom, vec(dom, k), bcs).log_coefficient_gradient(vec(dom, lam), vec(dom, u), g)
+    assert rel_err(g.download(), om.log_k_gradient(k, lam, u, *bcs)) < 1e-12
