@@ -1428,11 +1428,12 @@ template <typename T> void div_impl(tng_operator &op, const tng_vector &src, tng
     a.bc_cmb = op.bc_cmb; a.bc_surf = op.bc_surf;
     a.cidx = Index4(c.nx - 1, c.nr - 1);
     a.fidx = Index4(f.nx - 1, f.nr - 1);
-    // one pass for 128 radial cells, and for 64 in FP32: workgroups of CW
+    // one pass for 64 and 128 radial cells (64 in FP64, level 6: 34 us + fix-up against
+    // 63 us of the three kernels below): workgroups of CW
     // coarse node columns (times 2 radial parts for 128 cells) and a chunk of
     // coarse rows, then the side contributions between workgroups
     const int ncr = f.nr - 1;
-    if ((ncr == 128 || (ncr == 64 && sizeof(T) == 4)) && f.nalloc < ((int64_t)1 << 31)) {
+    if ((ncr == 128 || ncr == 64) && f.nalloc < ((int64_t)1 << 31)) {
         constexpr int CW = TNG_DIV_CW;
         const int RW = ncr == 128 ? 2 : 1;
         DivSide sb{};
