@@ -56,9 +56,6 @@ template <typename T> struct ApplyArgs {
     T *dst0, *dst1, *dst2;
     const T *k;
     const T *radii;     // (nsd, nr)
-    // the same in FP64: a layer's thickness is the difference of two radii, of
-    // which FP32 values keep few digits (128 layers: 1e-5 relative)
-    const double *radii64;
     const T *latgeom;   // (nsd, nc, nc, 2, 10)
     const T *coords;    // (nsd, nx, nx, 3) unit vectors (the radial normal)
     const T *btab;      // (nsd, nx, nx, 2, 3) boundary rows
@@ -87,6 +84,9 @@ template <typename T> struct ApplyArgs {
     T *cd0, *cd1, *cd2, *cx0, *cx1, *cx2;
     T caz, cad;
     int cread_d;
+    // the radii in FP64 for FP32 applies: a layer's thickness is the difference
+    // of two radii, of which FP32 values keep few digits (128 layers: 1e-5 relative)
+    const double *radii64;
 };
 
 template <typename T> __device__ __forceinline__ void normal_of(const T *c, T n[3])
@@ -494,7 +494,14 @@ __global__ __launch_bounds__(NW * 64) void epsdivdiv_apply_kernel(const ApplyArg
     #pragma unroll
         for (int p = 0; p < K; ++p) {
             const int l = lvl0 + p;
-            const double r0 = a.radii64[(int64_t)sd * nr + l], r1 = a.radii64[(int64_t)sd * nr + l + 1];
+            double r0, r1;
+            if constexpr (sizeof(T) == 8) {
+                r0 = a.radii[(int64_t)sd * nr + l];
+                r1 = a.radii[(int64_t)sd * nr + l + 1];
+            } else {
+                r0 = a.radii64[(int64_t)sd * nr + l];
+                r1 = a.radii64[(int64_t)sd * nr + l + 1];
+            }
             const double rmid = 0.5 * (r0 + r1), h = 0.5 * (r1 - r0);
             const double hs = 0.5 / rmid, tt = 1.0 / (6.0 * h);
             qq[p] = (T)(tt / hs);
