@@ -451,8 +451,8 @@ __global__ __launch_bounds__(64) void cpcg_boundary_kernel(const CpcgArgs a)
     for (int e = 0; e < 9; ++e) row[e * W] = B[e / 3][e % 3] + (u == v ? ann * nu_[e / 3] * nu_[e % 3] : 0.0);
 }
 
-// state: iteration count, done flag, first residual norm, total iterations,
-// then r.r of iteration 0, 1, ... (kHist slots, used in turn)
+// state: iteration count, the launch that ended the solve (0 while it runs),
+// first residual norm, total iterations, then r.r in two slots used in turn
 enum { CS_ITERS = 0, CS_DONE, CS_INIT, CS_TOTAL, CS_RR, CS_N = CS_RR + 2 };
 constexpr int kCpcgNodes = 16;    // nodes per block of the matrix kernel: 16 lanes each
 constexpr int kCpcgMaxParts = 1024;
@@ -471,6 +471,17 @@ __device__ __forceinline__ double parts_sum(const double *p, int n, double *red)
     double v = 0.0;
     for (int i = threadIdx.x; i < n; i += 256) v += p[i];
     return block_sum256(v, red);
+}
+
+// Launch numbers within a solve: 2 it for the matrix kernel of iteration it,
+// 2 it + 1 for the update kernel.  The block that ends the solve records the
+// number while other blocks of the launch may still be reading it: only an
+// earlier launch's number ends a block here, so that all threads of a block,
+// whichever value they saw, reach the block sums and take the decision there.
+__device__ __forceinline__ bool cpcg_ended_before(const double *st, int launch)
+{
+    const double done = st[CS_DONE];
+    return done != 0.0 && done < (double)launch;
 }
 
 // r = b, p = 0, x = 0; partials of r.r
@@ -507,7 +518,7 @@ __global__ __launch_bounds__(256) void cpcg_matrix_kernel(const double *A, const
                                                           double atol)
 {
     __shared__ double red[4];
-    if (st[CS_DONE] != 0.0) return;  // written by an earlier launch
+    if (cpcg_ended_before(st, 2 * it)) return;
     constexpr int W = CoarsePcg::kWidth;
     const int u = blockIdx.x * kCpcgNodes + (threadIdx.x >> 4), lane = threadIdx.x & 15;
     int v[2];
@@ -526,7 +537,7 @@ __global__ __launch_bounds__(256) void cpcg_matrix_kernel(const double *A, const
             const double init = sqrt(rr);
             st[CS_INIT] = init;
             st[CS_RR + 1] = rr;
-            if (init < atol) st[CS_DONE] = 1.0;
+            if (init < atol) st[CS_DONE] = 2 * it;
         }
         if (sqrt(rr) < atol) return;
     } else {
@@ -536,7 +547,7 @@ __global__ __launch_bounds__(256) void cpcg_matrix_kernel(const double *A, const
             st[CS_RR + (it & 1)] = rr;
             st[CS_ITERS] = it - 1;
             if (stop) {
-                st[CS_DONE] = 1.0;
+                st[CS_DONE] = 2 * it;
                 st[CS_TOTAL] += it - 1;
             }
         }
@@ -575,14 +586,14 @@ __global__ __launch_bounds__(256) void cpcg_update_kernel(int n, double *x, doub
                                                           int it, int max_it)
 {
     __shared__ double red[4];
-    if (st[CS_DONE] != 0.0) return;
+    if (cpcg_ended_before(st, 2 * it + 1)) return;
     const double pap = parts_sum(pparts, npp, red);
     const bool stop = fabs(pap) < DBL_MIN;
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t == 0 && (stop || it == max_it)) {
         st[CS_ITERS] = it;
         st[CS_TOTAL] += it;
-        if (stop) st[CS_DONE] = 1.0;
+        if (stop) st[CS_DONE] = 2 * it + 1;
     }
     if (stop) return;
     const double alpha = st[CS_RR + (it & 1)] / pap;

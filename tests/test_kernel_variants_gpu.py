@@ -85,6 +85,27 @@ def test_assembled_coarse_pcg_solves_the_coarse_system(bcs, gca, sdr, dtype, gpu
     assert rel_err(out[1], out[0]) < (1e-8 if dtype == tng.F64 else 1e-6)
 
 
+# launches after the end of a coarse solve change nothing, wherever in the host's look at the end (every 25) it falls:
+# ended by the tolerance within the first 25 iterations, and by a zero right-hand side, for which p.(A p) is zero
+@pytest.mark.parametrize("dtype", [tng.F64, tng.F32])
+def test_coarse_pcg_keeps_its_result_after_the_end(dtype, gpu_ctx):
+    om = O.Mesh(3, 3)
+    eta, b = np.exp(0.5 * field(om, 1, 13)), field(om, 3, 14)
+    out, zero = [], []
+    for max_it in (24, 25, 26, 400):
+        S = tng.StokesSolver(2, 3, 0.55, 1.0, (D, D), tng.StokesParams.defaults(
+            viscous_pc_dtype=dtype, coarse_max_iterations=max_it, coarse_relative_tolerance=1e-2,
+            coarse_absolute_tolerance=0.0))
+        dv = S.domain_velocity
+        S.set_viscosity(vec(dv, eta))
+        for rhs, res in ((b, out), (0 * b, zero)):
+            x = tng.VectorQ1Vec(dv)
+            S.precondition_velocity(x, vec(dv, rhs))
+            res.append(x.download())
+    assert np.any(out[0]) and all(np.array_equal(o, out[0]) for o in out)
+    assert all(not np.any(z) for z in zero)
+
+
 # the fan kernel: every lane-group size (4 to 32 layers; 32 in FP32 only, FP64 takes the sweep there), shared nodes of
 # two to five copies inside and across diamonds, every boundary mix, Add mode and skipped communication
 @pytest.mark.parametrize("L,Lr,ls", [(2, 2, 1), (3, 3, 2), (3, 4, 1), (4, 5, 0), (1, 3, 0), (5, 2, 2)])
