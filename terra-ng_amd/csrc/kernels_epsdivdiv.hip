@@ -1576,7 +1576,7 @@ void apply_impl(tng_operator &op, const tng_vector &src, tng_vector &dst, hipStr
     hipEvent_t *ev = ctx.profiling && !ws ? ctx.prof_next_set() : nullptr;
     if (ev) TNG_HIP_CHECK(hipEventRecord(ev[0], s));
     if (fan_applies(op)) {
-        // 4 to 32 radial layers without penalty: one launch, halo sum included
+        // small meshes without penalty: one launch, halo sum included
         if (!op.btab_valid) epsdivdiv_update_boundary_table(op, s);
         if (ev) TNG_HIP_CHECK(hipEventRecord(ev[1], s));
         fan_apply(op, src, dst, s);

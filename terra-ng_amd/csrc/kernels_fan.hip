@@ -1,5 +1,5 @@
-// EpsilonDivDiv apply for subdomains of 4 to 32 radial layers (the small
-// multigrid levels and small meshes), halo sum and Chebyshev sub-step
+// EpsilonDivDiv apply for meshes of 4 to 32 radial layers that do not fill the
+// chip (fan_pays; the small multigrid levels), halo sum and Chebyshev sub-step
 // included: one launch for what the sweeping apply, the halo sum and the
 // vector update do in three (the discretisation and its references are those
 // of kernels_epsdivdiv.hip).  Sub-step of the smoother, FP32 no-slip: level 3
@@ -367,13 +367,48 @@ template <typename T, int MODE> void fan_launch(const tng_domain &m, const FanAr
 
 }  // namespace
 
+// The fan evaluates a triangle three times, the sweep (with its halo sum) once
+// but as a serial loop over the rows of a strip, whose lanes may reach past
+// narrow subdomains.  Measured at lateral levels 2 to 10, diamonds whole and
+// split up to 16 x 16 (fan against sweep, no-slip):
+//   lanes F <= 2^20, one filling of the chip: the fan always (FP64 level 4, 16
+//     layers 7.6 against 13.9 us, level 6, 8 layers 30 against 35; FP32 level 5,
+//     32 layers 14.7 against 23.3);
+//   more: against the sweep's lanes times steps S.  FP64 from S = 2 F on
+//     (level 7, 8 layers: S / F = 0.76 105 against 79 us, 2.2 121 against 150;
+//     level 6, 16 layers: 0.77 56 against 43, 1.08 62 against 51, 2.3 70 against
+//     86); 4 layers, where the sweep fills its strips badly, up to 2^23
+//     (level 8 256 against 306, level 9 with free slip 1193 against 1081);
+//   FP32, 4 layers: always (level 9 412 against 839 us).  Up to 2^21 lanes, 8
+//     layers without free slip at any size, from S = 0.75 F on, with the free-slip
+//     projections of every column it reads from S = F on (level 6, 16 layers: 0.77
+//     21.5 against 24.3, free slip 26.2 against 25.9, 1.04 22.6 against 29.7 and
+//     27.1 against 31.3; level 7, 8 layers: 0.76 43.8 against 50.2, free slip 54.3
+//     against 53.2); else from S = 2 F on (level 6, 32 layers: 0.64 47.7
+//     against 34.6; level 7, 16 layers: 0.63 81 against 57).
+// Sub-steps of the smoother divide the same way: with the update kernel that
+// the fan spares, V-cycles on level 6, 8 layers gain 1.46 (FP32) and 1.03 (FP64),
+// level 6, 16 layers with free slip lose 0.94 and 0.75.  FP64 at 32 layers
+// always takes the sweep: 174 to 216 registers leave two waves per SIMD, and 21,780
+// groups of three triangles take 44 us at level 5 against 28 us.
+bool fan_pays(const tng_domain &m, bool f32, bool free_slip)
+{
+    const int cells = m.nr - 1;
+    if (m.rad_sdr != 0 || cells < 4 || cells > (f32 ? 32 : 16)) return false;
+    const double fan = 2.0 * cells * (double)m.nlat;
+    if (fan <= 1 << 20) return true;
+    // workgroups of eight waves take 512 / cells - 1 new columns of one subdomain
+    const int columns = 512 / cells - 1, strips = (m.nx + columns - 1) / columns;
+    const double sweep = 512.0 * m.nsd * strips * (m.nx + 2.5);
+    if (cells == 4 && (f32 || fan <= 1 << 23)) return true;
+    if (f32 && (fan <= 1 << 21 || (cells == 8 && !free_slip))) return sweep >= (free_slip ? 1.0 : 0.75) * fan;
+    return sweep >= 2.0 * fan;
+}
+
 bool fan_applies(const tng_operator &op)
 {
-    // FP64 at 32 layers stays with the sweep: 174-216 registers leave two waves
-    // per SIMD, and 10,890 groups of three triangles then take 44 us at level 5
-    // against 28 us for the sweep and its halo sum
-    return op.mesh->fan_blocks > 0 && !op.stored && !op.diagonal && !op.penalty_active &&
-           (op.mesh->nr - 1 <= 16 || op.k->dtype == TNG_F32);
+    if (op.mesh->fan_blocks == 0 || op.stored || op.diagonal || op.penalty_active) return false;
+    return fan_pays(*op.mesh, op.k->dtype == TNG_F32, op.bc_cmb == TNG_FREESLIP || op.bc_surf == TNG_FREESLIP);
 }
 
 void fan_apply(tng_operator &op, const tng_vector &src, tng_vector &dst, hipStream_t s)

@@ -208,14 +208,13 @@ void mesh_build(tng_domain &m, int lat_level, int rad_level, double r_min, doubl
     // task table of the fan apply: groups of copies in the order of their first
     // column, none across two blocks
     const int ncr = nr - 1;
-    if (rad_sdr == 0 && ncr >= 4 && ncr <= 32) {
+    if (fan_pays(m, true, false) || fan_pays(m, false, false)) {
         const int cap = (ncr == 32 ? 512 : 256) / (2 * ncr);  // as kFanCap
-        std::vector<int64_t> order;
-        for (size_t g = 0; g < lat_groups.size(); ++g) order.push_back((int64_t)g);
-        std::sort(order.begin(), order.end(),
-                  [&](int64_t a, int64_t b) { return lat_groups[a].front() < lat_groups[b].front(); });
-        for (const int64_t g : order) {
-            const auto &cols = lat_groups[g];  // ascending (sorted keys carry the column)
+        m.fan_col.reserve((size_t)m.nlat + m.nlat / 8);
+        m.fan_grp.reserve((size_t)m.nlat + m.nlat / 8);
+        for (int64_t c0 = 0; c0 < m.nlat; ++c0) {
+            const auto &cols = lat_groups[lat_id[c0]];  // ascending (sorted keys carry the column)
+            if (cols.front() != c0) continue;
             TNG_REQUIRE((int)cols.size() <= cap, "more copies of a lateral node than a block holds");
             const int used = (int)(m.fan_col.size() % cap);
             if (used + (int)cols.size() > cap) {

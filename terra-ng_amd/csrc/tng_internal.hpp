@@ -311,8 +311,9 @@ void epsdivdiv_apply_noalloc(tng_operator &op, const tng_vector &src, tng_vector
 bool epsdivdiv_apply_cheb(tng_operator &op, const tng_vector &x, tng_vector &ax, tng_vector &x_out, tng_vector &d,
                           const tng_vector &b, const tng_vector &invd, double az, double ad, bool read_d,
                           hipStream_t s);
-// The same for 4 to 32 radial layers in one launch (kernels_fan.hip): apply,
+// The same for few radial layers on a small mesh in one launch (kernels_fan.hip): apply,
 // halo sum and, in the second, the sub-step.
+bool fan_pays(const tng_domain &m, bool f32, bool free_slip);  // where it is the faster path
 bool fan_applies(const tng_operator &op);
 void fan_apply(tng_operator &op, const tng_vector &src, tng_vector &dst, hipStream_t s);
 void fan_apply_cheb(tng_operator &op, const tng_vector &x, tng_vector &x_out, tng_vector &d, const tng_vector &b,

@@ -1,6 +1,8 @@
 """Kernel variants at the sizes where their decompositions change: against
 the oracle at 1e-12 (FP64: sums of at most a few hundred products of one
 sign-free magnitude, 1e-16 each)."""
+import time
+
 import numpy as np
 import pytest
 
@@ -128,6 +130,44 @@ def test_fan_apply_matches_oracle(L, Lr, ls, bcs, gpu_ctx):
             op.apply(uv, out)
             ref = om.epsdivdiv(k, u, *bcs, apply_mode=mode[0], comm=mode[1], dst=base)
             assert rel_err(out.download(), ref) < tol
+
+
+def microseconds(dom, fn, n=20):
+    best = 1e9
+    for _ in range(5):
+        dom.ctx.synchronize()
+        t = time.perf_counter()
+        for _ in range(n):
+            fn()
+        dom.ctx.synchronize()
+        best = min(best, (time.perf_counter() - t) / n)
+    return 1e6 * best
+
+
+# wide meshes of few layers: the fan kernel's triple evaluation must not be taken there.  The rotation penalty of free
+# slip on both surfaces always takes the sweep, and does strictly more than an apply without it
+@pytest.mark.parametrize("L,Lr,dtype", [(7, 4, tng.F64), (7, 3, tng.F64), (7, 5, tng.F32), (7, 4, tng.F32)])
+def test_wide_meshes_take_no_longer_than_with_the_penalty(L, Lr, dtype, gpu_ctx):
+    dom = tng.DistributedDomain.create_uniform(L, Lr, 0.55, 1.0)
+    k, u, out = tng.VectorQ1Scalar(dom, dtype), tng.VectorQ1Vec(dom, dtype), tng.VectorQ1Vec(dom, dtype)
+    k.fill(1.0)
+    u.fill(1.0)
+    ops = [tng.EpsilonDivDivKerngen(dom, k, bcs) for bcs in ((D, F), (F, F))]
+    ops[1].set_penalty_epsilon(1.0)
+    plain, penalised = (microseconds(dom, lambda op=op: op.apply(u, out)) for op in ops)
+    assert plain < penalised
+
+
+# both sides of the line, and meshes whose narrow subdomains move it
+@pytest.mark.parametrize("L,Lr,ls", [(6, 4, 0), (6, 4, 3), (7, 2, 0), (6, 5, 0)])
+def test_fan_and_sweep_on_wide_meshes_match_oracle(L, Lr, ls, gpu_ctx):
+    dom, om = tng.DistributedDomain.create_uniform(L, Lr, 0.55, 1.0, ls, 0), O.Mesh(L, Lr, 0.55, 1.0, ls, 0)
+    k, u = np.exp(0.5 * field(om, 1, 36)), field(om, 3, 37)
+    ref = om.epsdivdiv(k, u, D, F)
+    for dtype, tol in ((tng.F64, 1e-12), (tng.F32, 1e-6)):  # FP32: operands and tables rounded to 6e-8, sums of 36 terms
+        out = tng.VectorQ1Vec(dom, dtype)
+        tng.EpsilonDivDivKerngen(dom, vec(dom, k, dtype), (D, F)).apply(vec(dom, u, dtype), out)
+        assert rel_err(out.download(), ref) < tol
 
 
 # copies that differ (a vector that no exchange has made consistent): each copy's cells read their own subdomain's values
