@@ -323,13 +323,15 @@ StokesSolver::StokesSolver(tng_context *ctx, int min_level, int max_level, int r
     }
     mg.pre.resize(nl);
     mg.post.resize(nl);
-    // spare solution vectors for the fused Chebyshev sub-steps (one-column
-    // apply kernels: 64 or 128 radial cells; the fan kernel: 4 to 32); the
-    // cheb_fuse setting 0 turns them off
+    // spare solution vectors for the fused Chebyshev sub-steps of the smoothed
+    // levels that take them (one-column apply kernels: 64 or 128 radial cells;
+    // the fan kernel where it applies; not stored matrices); the cheb_fuse
+    // setting 0 turns them off
     const bool fuse = vel->ctx->tuning.cheb_fuse != 0;
-    for (int l = 0; l < nl; ++l) {
+    for (int l = 1; l < nl; ++l) {
         const int ncells = meshes[l]->nr - 1;
-        if (fuse && l > 0 && (ncells == 64 || ncells == 128 || meshes[l]->fan_blocks > 0) && meshes[l]->rad_sdr == 0)
+        const bool takes = ncells == 64 || ncells == 128 || fan_applies(*mg.levels[l].A);
+        if (fuse && takes && !galerkin_level(l) && meshes[l]->rad_sdr == 0)
             mg.pre[l].xb = mg.post[l].xb = vec(pool, meshes[l].get(), mgt, 3);
     }
     for (int l = 0; l < nl; ++l)

@@ -1,6 +1,7 @@
 """Kernel variants at the sizes where their decompositions change: against
 the oracle at 1e-12 (FP64: sums of at most a few hundred products of one
 sign-free magnitude, 1e-16 each)."""
+import ctypes
 import time
 
 import numpy as np
@@ -197,6 +198,23 @@ def test_fan_chebyshev_has_the_bits_of_the_separate_kernels(dtype, bcs, sdr, gpu
             S.precondition_velocity(x, vec(S.domain_velocity, b))
         out.append(x.download())
     assert np.array_equal(out[0], out[1])
+
+
+# spare vectors of the fused sub-step only where a level takes it: none with the rotation penalty below 64 layers
+def test_no_spare_vectors_where_no_sub_step_is_fused(gpu_ctx):
+    def free_memory():
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert tng.load_library().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    used = []
+    for fuse in (0, 1):
+        free = free_memory()
+        with tng.default_context().tuning(cheb_fuse=fuse):
+            S = tng.StokesSolver(2, 5, 0.55, 1.0, (F, F), tng.StokesParams.defaults(krylov_restart=2))
+        used.append(free - free_memory())
+        S.close()
+    assert used[1] - used[0] < 4 << 20  # one vector of the finest level is 8.6 MB
 
 
 # FP32 at 128 layers, two cells per lane: strips of eight columns within one subdomain and across several, every
