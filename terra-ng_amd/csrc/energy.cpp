@@ -222,7 +222,7 @@ void energy_step(tng_energy_s &e, double dt, tng_solve_report &rep)
     // diagonal once for all its applies
     const tng_domain &m = *e.temp->mesh;
     if (!e.tau.p) e.tau.alloc(supg_tau_count(m) * sizeof(double));
-    if (!e.bdiag.p) e.bdiag.alloc(2 * (size_t)m.nlat * sizeof(double));
+    if (!e.bdiag.p) e.bdiag.alloc(supg_boundary_count(m) * sizeof(double));
     struct StepData {
         tng_operator *ops[3];
         StepData(tng_energy_s &e) : ops{e.A.get(), e.A_neumann.get(), e.A_neumann_diag.get()}

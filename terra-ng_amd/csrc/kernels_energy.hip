@@ -57,11 +57,15 @@ struct SupgArgs {
     const double *coords, *radii;
     const uint8_t *sd_cmb, *sd_surf;
     const double *tau;    // (cell, wedge), nullptr: no streamline term
-    const double *bdiag;  // (lateral node, side): diagonal entries of the treated boundary rows
+    // (lateral cell, side, corner): its share of the treated boundary rows'
+    // diagonal entries, read by the gather (bdiag) and written (bshare)
+    const double *bdiag;
+    double *bshare;
     double *partial;      // (lateral cell, corner, level)
     double *dst;
     double kappa, dt, mass;
     int treat_boundary, lumped, add;
+    int bblocks;    // blocks of the cell kernel's grid that form bshare
     int nsd, nx, nr;
     int lr, lc;     // log2 of the radial and lateral cells per subdomain
     int plen, lseg; // entries per (lateral cell, corner), log2 of the cells per radial segment
@@ -74,8 +78,13 @@ struct SupgGeom {
     double m2[3], g22, det;
 };
 
-// Fills entry (w, s) of the geometry of lateral cell col.
-__device__ __forceinline__ void supg_geometry(const SupgArgs &a, int64_t col, int w, int s, SupgGeom &G)
+// The same at one point.
+struct SupgPoint {
+    double m0[3], m1[3], m2[3], g00, g01, g11, g02, g12, g22, det;
+};
+
+// Wedge w of lateral cell col at lateral point s.
+__device__ __forceinline__ SupgPoint supg_point(const SupgArgs &a, int64_t col, int w, int s)
 {
     const int nc = a.nx - 1;
     const int yc = (int)(col & (nc - 1)), xc = (int)((col >> a.lc) & (nc - 1)), sd = (int)(col >> (2 * a.lc));
@@ -98,27 +107,43 @@ __device__ __forceinline__ void supg_geometry(const SupgArgs &a, int64_t col, in
         o[2] = x[0] * y[1] - x[1] * y[0];
     };
     auto dot = [](const double *x, const double *y) { return x[0] * y[0] + x[1] * y[1] + x[2] * y[2]; };
-    double n[3], m0[3], m1[3];
-    cross(e1, e2, n);
-    cross(e2, p, m0);
-    cross(p, e1, m1);
-    const double det = dot(n, p), id = 1.0 / det;
+    SupgPoint g;
+    cross(e1, e2, g.m2);
+    cross(e2, p, g.m0);
+    cross(p, e1, g.m1);
+    const double det = dot(g.m2, p), id = 1.0 / det;
     for (int d = 0; d < 3; ++d) {
-        n[d] *= id;
-        m0[d] *= id;
-        m1[d] *= id;
-        G.m0[s][d] = m0[d];
-        G.m1[s][d] = m1[d];
-        if (s == 0) G.m2[d] = n[d];
+        g.m2[d] *= id;
+        g.m0[d] *= id;
+        g.m1[d] *= id;
     }
-    G.g00[s] = dot(m0, m0);
-    G.g01[s] = dot(m0, m1);
-    G.g11[s] = dot(m1, m1);
-    G.g02[s] = dot(m0, n);
-    G.g12[s] = dot(m1, n);
+    g.g00 = dot(g.m0, g.m0);
+    g.g01 = dot(g.m0, g.m1);
+    g.g11 = dot(g.m1, g.m1);
+    g.g02 = dot(g.m0, g.m2);
+    g.g12 = dot(g.m1, g.m2);
+    g.g22 = dot(g.m2, g.m2);
+    g.det = fabs(det);
+    return g;
+}
+
+// Fills entry (w, s) of the geometry of lateral cell col.
+__device__ __forceinline__ void supg_geometry(const SupgArgs &a, int64_t col, int w, int s, SupgGeom &G)
+{
+    const SupgPoint g = supg_point(a, col, w, s);
+    for (int d = 0; d < 3; ++d) {
+        G.m0[s][d] = g.m0[d];
+        G.m1[s][d] = g.m1[d];
+        if (s == 0) G.m2[d] = g.m2[d];
+    }
+    G.g00[s] = g.g00;
+    G.g01[s] = g.g01;
+    G.g11[s] = g.g11;
+    G.g02[s] = g.g02;
+    G.g12[s] = g.g12;
     if (s == 0) {
-        G.g22 = dot(n, n);
-        G.det = fabs(det);
+        G.g22 = g.g22;
+        G.det = g.det;
     }
 }
 
@@ -280,6 +305,75 @@ __device__ __forceinline__ SupgCell supg_cell_of(const SupgArgs &a, int64_t cell
     return c;
 }
 
+// One wedge of a lateral cell at one surface (thread = (cell, side, wedge)): the
+// diagonal entries of its three corners there, summed over the cell's two
+// wedges into its four corner columns.
+__device__ __forceinline__ void supg_boundary(const SupgArgs &a, int64_t t)
+{
+    const int64_t ncol = a.ncell >> a.lr;
+    if (t >= 4 * ncol) return;
+    const int w = (int)(t & 1), side = (int)((t >> 1) & 1), nx = a.nx, nr = a.nr, nc = nx - 1;
+    const int64_t col = t >> 2;
+    const int yc = (int)(col & (nc - 1)), xc = (int)((col >> a.lc) & (nc - 1)), sd = (int)(col >> (2 * a.lc));
+    if ((side == 0 ? a.sd_cmb[sd] : a.sd_surf[sd]) == 0) return;  // not read there
+    const int rc = side == 0 ? 0 : nr - 2;
+    const double r1 = a.radii[(int64_t)sd * nr + rc], r2 = a.radii[(int64_t)sd * nr + rc + 1];
+    double ub[3][3], ut[3][3], out[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        const int64_t i = (((int64_t)sd * nx + xc + kEW[w][j][0]) * nx + yc + kEW[w][j][1]) * nr + rc;
+        ub[0][j] = a.u0[i];
+        ub[1][j] = a.u1[i];
+        ub[2][j] = a.u2[i];
+        ut[0][j] = a.u0[i + 1];
+        ut[1][j] = a.u1[i + 1];
+        ut[2][j] = a.u2[i + 1];
+    }
+    const double tau = a.tau ? a.tau[2 * ((col << a.lr) + rc) + w] : 0.0;
+    const double gr = 0.5 * (r2 - r1), igr = 1.0 / gr;
+    // a real loop: unrolled, three points' geometry is live at once
+#pragma unroll 1
+    for (int s = 0; s < 3; ++s) {
+        const int ks = s == 0 ? 1 : (s == 1 ? 2 : 0);
+        const SupgPoint g = supg_point(a, col, w, s);
+#pragma unroll
+        for (int z = 0; z < 2; ++z) {
+            const double zeta = z == 0 ? -kGauss : kGauss;
+            const double n0 = 0.5 * (1.0 - zeta), n1 = 0.5 * (1.0 + zeta);
+            const double r = r1 + gr * (1.0 + zeta), ir = 1.0 / r, wz = g.det * r * r * gr * (1.0 / 6.0);
+            double u[3];
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                const double z0 = n0 * ub[d][0] + n1 * ut[d][0], z1 = n0 * ub[d][1] + n1 * ut[d][1],
+                             z2 = n0 * ub[d][2] + n1 * ut[d][2];
+                u[d] = (z0 + z1 + z2) * (1.0 / 6.0) + 0.5 * (ks == 0 ? z0 : (ks == 1 ? z1 : z2));
+            }
+            const double al = (u[0] * g.m0[0] + u[1] * g.m0[1] + u[2] * g.m0[2]) * ir;
+            const double be = (u[0] * g.m1[0] + u[1] * g.m1[1] + u[2] * g.m1[2]) * ir;
+            const double ga = (u[0] * g.m2[0] + u[1] * g.m2[1] + u[2] * g.m2[2]) * igr;
+            const double h00 = g.g00 * ir * ir, h01 = g.g01 * ir * ir, h11 = g.g11 * ir * ir, h02 = g.g02 * ir * igr,
+                         h12 = g.g12 * ir * igr, h22 = g.g22 * igr * igr;
+            const double nr_ = side == 0 ? n0 : n1, dr = side == 0 ? -0.5 : 0.5;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const double nl = k == ks ? 2.0 / 3.0 : 1.0 / 6.0;
+                const double lx = k == 0 ? -1.0 : (k == 1 ? 1.0 : 0.0), ly = k == 0 ? -1.0 : (k == 2 ? 1.0 : 0.0);
+                const double fx = lx * nr_, fy = ly * nr_, fz = nl * dr, phi = nl * nr_;
+                const double ug = fx * al + fy * be + fz * ga;
+                const double gg = fx * fx * h00 + fy * fy * h11 + fz * fz * h22 +
+                                  2.0 * (fx * fy * h01 + fx * fz * h02 + fy * fz * h12);
+                out[k] += wz * (a.mass * (a.lumped ? phi : phi * phi) + a.dt * (a.kappa * gg + ug * phi + tau * ug * ug));
+            }
+        }
+    }
+    // corner columns 00, 10, 01, 11: the first wedge's corners are 0, 1, 2, the
+    // second's 3, 2, 1.  The wedges sit in neighbouring lanes.
+    const double other = __shfl_xor(out[2], 1, 64);
+    double *o = a.bshare + (col * 2 + side) * 4;
+    o[w == 0 ? 0 : 3] = out[0];
+    o[w == 0 ? 1 : 2] = out[1] + other;
+}
+
 // One thread per cell (lanes along r), its two wedges together: the eight
 // nodes are loaded once, the lateral data of the block's columns is formed
 // once per block in LDS.  A corner column's contributions to a node level (the
@@ -290,13 +384,22 @@ __device__ __forceinline__ SupgCell supg_cell_of(const SupgArgs &a, int64_t cell
 // cells): 167 us + 24 us for the gather, against 721 us + 140 us with the
 // Jacobian inverse, tau and every row's diagonal formed at each of the six
 // points of each wedge and twelve partials per cell; tau takes 257 us, once
-// per step.
-template <bool DIAG> __global__ __launch_bounds__(256) void supg_cell_kernel(const SupgArgs a)
+// per step.  BND: the first blocks form the treated boundary rows' diagonal (an
+// apply outside an energy step).  In the cells' waves every lane would wait for
+// the boundary lanes; as a kernel of its own it cannot overlap, and one thread
+// per node and side, which evaluates each wedge three times, took 24 us at level
+// 4 and 250 us at level 7, 2 layers (a wedge once, in this launch: 1 and 35 us).
+template <bool DIAG, bool BND> __global__ __launch_bounds__(256) void supg_cell_kernel(const SupgArgs a)
 {
     extern __shared__ double smem[];
     const int tb_ = blockDim.x, ncr = 1 << a.lr;
     SupgGeom *geom = reinterpret_cast<SupgGeom *>(smem);
-    const int64_t cell0 = (int64_t)blockIdx.x * tb_, ncol = a.ncell >> a.lr;
+    if constexpr (BND)
+        if ((int)blockIdx.x < a.bblocks) {
+            supg_boundary(a, (int64_t)blockIdx.x * tb_ + threadIdx.x);
+            return;
+        }
+    const int64_t cell0 = (int64_t)(blockIdx.x - (BND ? a.bblocks : 0)) * tb_, ncol = a.ncell >> a.lr;
     const int64_t col0 = cell0 >> a.lr;
     const int cols = tb_ > ncr ? tb_ >> a.lr : 1;
     double *tops = smem + cols * 2 * (sizeof(SupgGeom) / sizeof(double));  // (corner, thread)
@@ -410,10 +513,15 @@ __global__ __launch_bounds__(256) void supg_gather_kernel(const SupgArgs a, cons
         }
     }
     double s = (v[0] + v[1]) + (v[2] + v[3]);
-    if (a.bdiag) {
-        const uint32_t lcol = ((uint32_t)sd * a.nx + X) * a.nx + Y;
-        if (l == 0 && a.sd_cmb[sd]) s = a.bdiag[2 * lcol] * a.src[gid];
-        else if (l == ncr && a.sd_surf[sd]) s = a.bdiag[2 * lcol + 1] * a.src[gid];
+    if (a.bdiag && ((l == 0 && a.sd_cmb[sd]) || (l == ncr && a.sd_surf[sd]))) {
+        double b[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int xc = X - (k & 1), yc = Y - (k >> 1);
+            const bool in = xc >= 0 && xc < nc && yc >= 0 && yc < nc;
+            b[k] = in ? a.bdiag[((((int64_t)sd * nc + xc) * nc + yc) * 2 + (l == 0 ? 0 : 1)) * 4 + k] : 0.0;
+        }
+        s = ((b[0] + b[1]) + (b[2] + b[3])) * a.src[gid];
     }
     a.dst[gid] = a.add ? a.dst[gid] + s : s;
 }
@@ -463,50 +571,10 @@ __global__ __launch_bounds__(256) void supg_tau_kernel(const SupgArgs a, double 
     }
 }
 
-// Diagonal entries of the treated boundary rows, per lateral node copy and
-// side: one thread per entry, gathering over the wedges around it.
-__global__ __launch_bounds__(64) void supg_bdiag_kernel(const SupgArgs a, double *bdiag, int64_t n)
+// The boundary rows alone (an energy step forms them once for all its applies).
+__global__ __launch_bounds__(256) void supg_boundary_kernel(const SupgArgs a)
 {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    const int side = (int)(t & 1), nx = a.nx, nr = a.nr, nc = nx - 1;
-    const int64_t lcol = t >> 1;
-    const int Y = (int)(lcol % nx), X = (int)((lcol / nx) % nx), sd = (int)(lcol / ((int64_t)nx * nx));
-    double acc = 0.0;
-    if (side == 0 ? a.sd_cmb[sd] != 0 : a.sd_surf[sd] != 0) {
-        const int rc = side == 0 ? 0 : nr - 2;
-        const double r1 = a.radii[(int64_t)sd * nr + rc], r2 = a.radii[(int64_t)sd * nr + rc + 1];
-        for (int k = 0; k < 4; ++k) {
-            const int xc = X - (k & 1), yc = Y - (k >> 1);
-            if (xc < 0 || xc >= nc || yc < 0 || yc >= nc) continue;
-            const int64_t col = ((int64_t)sd * nc + xc) * nc + yc;
-            for (int w = 0; w < 2; ++w) {
-                // wedge corners as corner columns of the cell; the node is corner k
-                const int kc = w == 0 ? (k == 3 ? -1 : k) : (k == 0 ? -1 : 3 - k);
-                if (kc < 0) continue;
-                SupgGeom G;
-                for (int s = 0; s < 3; ++s) supg_geometry(a, col, w, s, G);
-                double ub[3][4], ut[3][4], db[3], dt_[3];
-                for (int j = 0; j < 3; ++j) {
-                    const int64_t i = (((int64_t)sd * nx + xc + kEW[w][j][0]) * nx + yc + kEW[w][j][1]) * nr + rc;
-                    ub[0][j] = a.u0[i];
-                    ub[1][j] = a.u1[i];
-                    ub[2][j] = a.u2[i];
-                    ut[0][j] = a.u0[i + 1];
-                    ut[1][j] = a.u1[i + 1];
-                    ut[2][j] = a.u2[i + 1];
-                }
-                const double tau = a.tau ? a.tau[2 * ((col << a.lr) + rc) + w] : 0.0;
-                supg_wedge_diag(a, &G, 0, ub, ut, r1, r2, tau, db, dt_);
-                double mb = 0.0, mt = 0.0;
-                if (a.lumped) supg_lumped_mass(a, G, r1, r2, mb, mt);
-                const double vb = kc == 0 ? db[0] : (kc == 1 ? db[1] : db[2]);
-                const double vt = kc == 0 ? dt_[0] : (kc == 1 ? dt_[1] : dt_[2]);
-                acc += side == 0 ? vb + mb : vt + mt;
-            }
-        }
-    }
-    bdiag[t] = acc;
+    supg_boundary(a, (int64_t)blockIdx.x * blockDim.x + threadIdx.x);
 }
 
 // g: the Dirichlet temperatures at the boundary nodes (CMB first), zero elsewhere
@@ -622,10 +690,12 @@ void supg_boundary_diagonal(const tng_operator &op, const double *tau, double *b
 {
     SupgArgs a = supg_args(op);
     a.tau = op.supg_enabled ? tau : nullptr;
-    const int64_t n = 2 * op.mesh->nlat;
-    hipLaunchKernelGGL(supg_bdiag_kernel, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, s, a, bdiag, n);
+    a.bshare = bdiag;
+    hipLaunchKernelGGL(supg_boundary_kernel, dim3(grid1d(4 * (a.ncell >> a.lr))), dim3(256), 0, s, a);
     TNG_HIP_CHECK(hipGetLastError());
 }
+
+size_t supg_boundary_count(const tng_domain &m) { return (size_t)m.nsd * (m.nx - 1) * (m.nx - 1) * 8; }
 
 size_t supg_tau_count(const tng_domain &m) { return (size_t)m.nsd * (m.nx - 1) * (m.nx - 1) * (m.nr - 1) * 2; }
 
@@ -636,7 +706,7 @@ void supg_apply(tng_operator &op, const tng_vector &src, tng_vector &dst, hipStr
     SupgArgs a = supg_args(op);
     // work space: corner partials, then (outside an energy step, which brings
     // its own) tau and the boundary diagonal of this apply's velocity
-    const size_t npart = (size_t)(a.ncell >> a.lr) * 4 * a.plen, ntau = supg_tau_count(m), nb = 2 * (size_t)m.nlat;
+    const size_t npart = (size_t)(a.ncell >> a.lr) * 4 * a.plen, ntau = supg_tau_count(m), nb = supg_boundary_count(m);
     const bool own_tau = op.supg_enabled && !op.supg_step_tau;
     const bool treat = op.supg_treat_boundary && !op.diagonal;
     const bool own_bdiag = treat && !op.supg_step_bdiag;
@@ -650,19 +720,24 @@ void supg_apply(tng_operator &op, const tng_vector &src, tng_vector &dst, hipStr
         if (own_tau) supg_tau(op, a.partial + npart, s);
         a.tau = own_tau ? a.partial + npart : op.supg_step_tau;
     }
-    if (treat) {
-        double *own = a.partial + npart + (own_tau ? ntau : 0);
-        if (own_bdiag) supg_boundary_diagonal(op, a.tau, own, s);
-        a.bdiag = own_bdiag ? own : op.supg_step_bdiag;
-    }
     const int tb = supg_block(1 << a.lr), cols = std::max(1, tb >> a.lr);
     const size_t lds = (size_t)cols * 2 * sizeof(SupgGeom) + (size_t)tb * 4 * sizeof(double);
-    const dim3 grid((unsigned)((a.ncell + tb - 1) / tb));
+    if (treat) {
+        double *own = a.partial + npart + (own_tau ? ntau : 0);
+        if (own_bdiag) {
+            a.bshare = own;
+            a.bblocks = (int)((4 * (a.ncell >> a.lr) + tb - 1) / tb);
+        }
+        a.bdiag = own_bdiag ? own : op.supg_step_bdiag;
+    }
+    const dim3 grid((unsigned)(a.bblocks + (a.ncell + tb - 1) / tb));
     if (op.diagonal) {
         a.treat_boundary = 0;  // every row keeps its own diagonal entry
-        hipLaunchKernelGGL(supg_cell_kernel<true>, grid, dim3(tb), lds, s, a);
+        hipLaunchKernelGGL((supg_cell_kernel<true, false>), grid, dim3(tb), lds, s, a);
+    } else if (a.bblocks > 0) {
+        hipLaunchKernelGGL((supg_cell_kernel<false, true>), grid, dim3(tb), lds, s, a);
     } else {
-        hipLaunchKernelGGL(supg_cell_kernel<false>, grid, dim3(tb), lds, s, a);
+        hipLaunchKernelGGL((supg_cell_kernel<false, false>), grid, dim3(tb), lds, s, a);
     }
     hipLaunchKernelGGL(supg_gather_kernel, dim3(grid1d(m.nalloc)), dim3(256), 0, s, a, Index4(m.nx, m.nr));
     TNG_HIP_CHECK(hipGetLastError());

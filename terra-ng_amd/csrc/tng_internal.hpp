@@ -384,9 +384,11 @@ void stored_apply(tng_operator &op, const tng_vector &src, tng_vector &dst, cons
 
 // energy equation (kernels_energy.hip, kernels_stokes.hip)
 void supg_apply(tng_operator &op, const tng_vector &src, tng_vector &dst, hipStream_t s);
-size_t supg_tau_count(const tng_domain &m);  // one tau per wedge
+size_t supg_tau_count(const tng_domain &m);       // one tau per wedge
+size_t supg_boundary_count(const tng_domain &m);  // lateral cells x 2 surfaces x 4 corners
 void supg_tau(const tng_operator &op, double *tau, hipStream_t s);
-void supg_boundary_diagonal(const tng_operator &op, const double *tau, double *bdiag, hipStream_t s);  // 2 nlat
+// the boundary rows' diagonal as shares of the lateral cells, which the gather sums
+void supg_boundary_diagonal(const tng_operator &op, const double *tau, double *bdiag, hipStream_t s);
 void launch_scalar_mass(const tng_vector &src, tng_vector &dst, hipStream_t s);
 void launch_boundary_values(tng_vector &g, double t_cmb, double t_surf, hipStream_t s);
 void launch_assign_masked(tng_vector &b, const tng_vector &src, uint8_t flag, hipStream_t s);

@@ -25,6 +25,18 @@ def vec(dom, data, dtype=tng.F64):
     return (tng.VectorQ1Vec if data.ndim == 5 else tng.VectorQ1Scalar)(dom, dtype).upload(data)
 
 
+def microseconds(dom, fn, n=20):
+    best = 1e9
+    for _ in range(5):
+        dom.ctx.synchronize()
+        t = time.perf_counter()
+        for _ in range(n):
+            fn()
+        dom.ctx.synchronize()
+        best = min(best, (time.perf_counter() - t) / n)
+    return 1e6 * best
+
+
 # columns per block of the SUPG cell kernel: 64 (2 and 4 cells), 32, one, and
 # radial segments of 256 cells whose seam levels two blocks share (512 layers)
 @pytest.mark.parametrize("L,Lr,ls,rs", [(2, 1, 0, 0), (3, 2, 1, 0), (2, 3, 0, 0), (2, 8, 0, 0), (1, 9, 0, 0), (1, 9, 0, 1)])
@@ -39,6 +51,20 @@ def test_supg_block_shapes(L, Lr, ls, rs, flags, gpu_ctx):
     ref = O.supg_apply(om, vel, T, kappa=0.01, dt=0.02, treat_boundary=flags.get("treat_boundary", True),
                        diagonal=flags.get("diagonal", False), lumped=flags.get("lumped_mass", False))
     assert rel_err(out.download(), ref) < 1e-12
+
+
+# the treated boundary rows must not cost more than a little beside the apply: the untreated diagonal mode has the same
+# kernels without them
+@pytest.mark.parametrize("L,Lr", [(4, 4), (6, 2), (5, 5)])
+def test_supg_boundary_rows_cost_little(L, Lr, gpu_ctx):
+    dom = tng.DistributedDomain.create_uniform(L, Lr, 0.55, 1.0)
+    v, t, out = tng.VectorQ1Vec(dom), tng.VectorQ1Scalar(dom), tng.VectorQ1Scalar(dom)
+    v.fill(1.0)
+    t.fill(1.0)
+    ops = [tng.UnsteadyAdvectionDiffusionSUPG(dom, v, 0.01, 0.02, **kw)
+           for kw in ({}, dict(diagonal=True, treat_boundary=False))]
+    treated, diagonal = (microseconds(dom, lambda op=op: op.apply(t, out)) for op in ops)
+    assert treated < 1.3 * diagonal
 
 
 def test_supg_reads_the_velocity_at_every_apply(gpu_ctx):
@@ -131,18 +157,6 @@ def test_fan_apply_matches_oracle(L, Lr, ls, bcs, gpu_ctx):
             op.apply(uv, out)
             ref = om.epsdivdiv(k, u, *bcs, apply_mode=mode[0], comm=mode[1], dst=base)
             assert rel_err(out.download(), ref) < tol
-
-
-def microseconds(dom, fn, n=20):
-    best = 1e9
-    for _ in range(5):
-        dom.ctx.synchronize()
-        t = time.perf_counter()
-        for _ in range(n):
-            fn()
-        dom.ctx.synchronize()
-        best = min(best, (time.perf_counter() - t) / n)
-    return 1e6 * best
 
 
 # wide meshes of few layers: the fan kernel's triple evaluation must not be taken there.  The rotation penalty of free
