@@ -1428,12 +1428,16 @@ template <typename T> void div_impl(tng_operator &op, const tng_vector &src, tng
     a.bc_cmb = op.bc_cmb; a.bc_surf = op.bc_surf;
     a.cidx = Index4(c.nx - 1, c.nr - 1);
     a.fidx = Index4(f.nx - 1, f.nr - 1);
-    // one pass for 64 and 128 radial cells (64 in FP64, level 6: 34 us + fix-up against
-    // 63 us of the three kernels below): workgroups of CW
+    // one pass for 64 and 128 radial cells: workgroups of CW
     // coarse node columns (times 2 radial parts for 128 cells) and a chunk of
-    // coarse rows, then the side contributions between workgroups
+    // coarse rows, then the side contributions between workgroups.  64 cells in
+    // FP64 below 2048 coarse cell columns keep the three kernels: a wave's
+    // serial sweep of two rows is longer than they are (level 3: 18.9 against
+    // 14.6 us, level 4, 640 columns, 19.2 against 17.0; level 5, 2560 columns,
+    // 22.0 against 29.8, level 6 46.7 against 75.4)
     const int ncr = f.nr - 1;
-    if ((ncr == 128 || ncr == 64) && f.nalloc < ((int64_t)1 << 31)) {
+    const bool small = sizeof(T) == 8 && ncr == 64 && (int64_t)c.nsd * (c.nx - 1) * (c.nx - 1) < 2048;
+    if ((ncr == 128 || ncr == 64) && !small && f.nalloc < ((int64_t)1 << 31)) {
         constexpr int CW = TNG_DIV_CW;
         const int RW = ncr == 128 ? 2 : 1;
         DivSide sb{};

@@ -214,6 +214,37 @@ def test_fan_chebyshev_has_the_bits_of_the_separate_kernels(dtype, bcs, sdr, gpu
     assert np.array_equal(out[0], out[1])
 
 
+# B and its transpose are adjoint: the one-pass divergence with chunks of 2, 4 and 8 coarse rows and the three kernels of
+# small FP64 meshes, at 64 layers per subdomain (random entries: a wrong one moves the product by 1e-7 or more of the
+# norms' product, rounding by a few 1e-16)
+@pytest.mark.parametrize("L,Lr,rs", [(4, 6, 0), (5, 6, 0), (7, 6, 0), (7, 7, 1)])
+def test_divergence_is_the_adjoint_of_the_gradient(L, Lr, rs, gpu_ctx):
+    fine, coarse = (tng.DistributedDomain.create_uniform(L - i, Lr - i, 0.55, 1.0, 0, rs) for i in range(2))
+
+    def noise(dom, k):  # the same on all copies of a node
+        s = (dom.coords() @ (1e3 * np.random.default_rng(k).uniform(1, 2, 3)))[..., None]
+        return np.sin(s + 1e4 * dom.radii()[:, None, None, :])
+
+    u = tng.VectorQ1Vec(fine).upload(np.stack([noise(fine, k) for k in range(3)]))
+    p = tng.VectorQ1Scalar(coarse).upload(noise(coarse, 3))
+    bu, btp = tng.VectorQ1Scalar(coarse), tng.VectorQ1Vec(fine)
+    tng.DivergenceKerngen(fine, coarse, (D, F)).apply(u, bu)
+    tng.GradientKerngen(fine, coarse, (D, F)).apply(p, btp)
+    assert abs(tng.dot(bu, p) - tng.dot(u, btp)) < 1e-13 * tng.norm_2(bu) * tng.norm_2(p)
+
+
+# the one-pass divergence's serial rows on small FP64 meshes: FP32, which takes it at every size, is the yardstick
+def test_small_divergence_takes_no_longer_in_fp64(gpu_ctx):
+    fine, coarse = (tng.DistributedDomain.create_uniform(3 - i, 6 - i, 0.55, 1.0) for i in range(2))
+    times = []
+    for dtype in (tng.F64, tng.F32):
+        u, out = tng.VectorQ1Vec(fine, dtype), tng.VectorQ1Scalar(coarse, dtype)
+        u.fill(1.0)
+        op = tng.DivergenceKerngen(fine, coarse, (D, F))
+        times.append(microseconds(fine, lambda: op.apply(u, out)))
+    assert times[0] < 1.05 * times[1]
+
+
 # spare vectors of the fused sub-step only where a level takes it: none with the rotation penalty below 64 layers
 def test_no_spare_vectors_where_no_sub_step_is_fused(gpu_ctx):
     def free_memory():
