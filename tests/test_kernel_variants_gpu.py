@@ -298,6 +298,41 @@ def test_fp32_pairs_fused_have_the_bits_of_the_separate_kernels(bcs, gpu_ctx):
     assert np.array_equal(out[0], out[1])
 
 
+# the same on split diamonds, and on a level that the last cache does not hold (the step's vectors pass by the caches)
+@pytest.mark.parametrize("L,extra,ls", [(4, 3, 1), (6, 1, 0)])
+def test_fp32_pairs_fused_split_and_streamed(L, extra, ls, gpu_ctx):
+    out, rng = [], np.random.default_rng(38)
+    for fuse in (0, 1):
+        with tng.default_context().tuning(cheb_fuse=fuse):
+            S = tng.StokesSolver(L - 1, L, 0.55, 1.0, (D, F), tng.StokesParams.defaults(
+                viscous_pc_dtype=tng.F32, viscous_pc_chebyshev_order=3, coarse_max_iterations=1, krylov_restart=2),
+                radial_extra_levels=extra, lateral_sdr=ls)
+        dv = S.domain_velocity
+        if not out:  # the same values on every copy of a node
+            s = dv.coords() @ (1e3 * rng.uniform(1, 2, (3, 4)))
+            noise = np.sin(np.moveaxis(s, -1, 0)[..., None] + 1e4 * dv.radii()[:, None, None, :])
+        S.set_viscosity(vec(dv, np.exp(0.5 * noise[3])))
+        x, b = tng.VectorQ1Vec(dv), vec(dv, noise[:3])
+        for _ in range(2):
+            S.precondition_velocity(x, b)
+        out.append(x.download())
+    assert np.any(out[0]) and np.array_equal(out[0], out[1])
+
+
+# a level that the last cache holds: the fused step is worth it only if it does not stream past that cache
+def test_fp32_pairs_fused_pay_on_a_cached_level(gpu_ctx):
+    times = []
+    for fuse in (0, 1):
+        with tng.default_context().tuning(cheb_fuse=fuse):
+            S = tng.StokesSolver(4, 5, 0.55, 1.0, (D, F), tng.StokesParams.defaults(
+                viscous_pc_dtype=tng.F32, viscous_pc_chebyshev_order=6, coarse_max_iterations=1, krylov_restart=2),
+                radial_extra_levels=2)
+        x, b = tng.VectorQ1Vec(S.domain_velocity), tng.VectorQ1Vec(S.domain_velocity)
+        b.fill(1.0)
+        times.append(microseconds(S.domain_velocity, lambda: S.precondition_velocity(x, b)))
+    assert times[1] < 0.96 * times[0]
+
+
 # the adjoint's wedge products: two layers (cells that meet at one node level), one and several rows per thread,
 # waves in one column (64 and 128 layers) and in several, radial subdomains without a boundary
 @pytest.mark.parametrize("L,Lr,ls,rs", [(1, 1, 0, 0), (2, 3, 1, 0), (2, 6, 0, 0), (1, 7, 0, 0), (3, 8, 0, 2), (5, 5, 0, 0),
