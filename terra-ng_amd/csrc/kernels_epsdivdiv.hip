@@ -1358,12 +1358,13 @@ struct ApplyShape {
     int R, K, RG, NW, S;
 };
 
-ApplyShape apply_shape(int ncells, const tng_tuning &tu, bool fused = false, bool f32 = false)
+// columns: node columns of the mesh
+ApplyShape apply_shape(int ncells, const tng_tuning &tu, int64_t columns, bool fused = false, bool f32 = false)
 {
     ApplyShape sh{64, 1, 1, 8, 1};
     const int chunks = tu.apply_radial_chunks;
     const bool split = tu.apply_radial_split != 0;
-    if (f32 && ncells == 128 && (fused ? chunks != 1 : chunks == 0 && split)) {
+    if (f32 && ncells == 128 && (fused ? chunks != 1 && columns >= 2048 : chunks == 0 && split)) {
         // FP32 is bound by vector instructions (a scalar FP32 operation costs
         // what an FP64 one does).  Two cells per lane issue a quarter fewer of
         // them than radial chunks or parts of 64 cells: strips of eight columns
@@ -1371,8 +1372,13 @@ ApplyShape apply_shape(int ncells, const tng_tuning &tu, bool fused = false, boo
         // the exchange and boundary terms serve two cells, and a lane moves its
         // levels as pairs.  10 x 129 x 129 columns: apply 312 us plus 15 us for
         // the levels between parts -> 240 us; fused Chebyshev sub-step 536 us
-        // (two chunks) -> 486 us.  FP64 takes 64 cells per lane set: two cells
-        // of it exceed the 256 registers that two waves per SIMD leave.
+        // (two chunks) -> 463 us.  Few columns leave CUs without a strip, and a
+        // wave's steps are longer: sub-step at 250 columns 18.6 us against 14.5
+        // with two chunks, 810 columns 20.6 against 15.4, 2890 columns 21.2 against
+        // 22.8.  An apply spares a launch: 250 columns 18.2 us against 18.0 in two
+        // parts (with the rotation penalty 26.6 against 27.4), 810 columns 18.6
+        // against 18.7, 2890 columns 19.0 against 19.3.  FP64 takes 64 cells per lane set: two cells of it exceed the 256
+        // registers that two waves per SIMD leave.
         sh.K = 2;
         return sh;
     }
@@ -1403,7 +1409,7 @@ template <typename T, bool FUSE = false> void launch_apply(ApplyArgs<T> a, hipSt
     // shapes: up to 64 radial cells one cell per lane (R lanes per column);
     // more as radial parts of 64 cells, or (128 and 256 cells) radial chunks
     // of one wave each or K cells per lane
-    const ApplyShape sh = apply_shape(a.ncells, tu, FUSE, sizeof(T) == 4);
+    const ApplyShape sh = apply_shape(a.ncells, tu, (int64_t)a.nsd * a.nx * a.nx, FUSE, sizeof(T) == 4);
     const int R = sh.R, K = sh.K, RG = sh.RG, NW = sh.NW;
     TNG_REQUIRE(K <= 4, "more than 256 radial layers per subdomain need the radial parts");
     a.rsplit = sh.S;
@@ -1441,13 +1447,11 @@ template <typename T, bool FUSE = false> void launch_apply(ApplyArgs<T> a, hipSt
             }
         }
     } else if (RG == 2) {
-        if constexpr (!FUSE || sizeof(T) == 8) {  // the fused step in FP32 takes two cells per lane
-            switch (bcm) {
-            case 0: launch_apply_rk<T, 64, 1, 8, 2, 0, FUSE>(a, lg, s, tu); break;
-            case 1: launch_apply_rk<T, 64, 1, 8, 2, 1, FUSE>(a, lg, s, tu); break;
-            case 2: launch_apply_rk<T, 64, 1, 8, 2, 2, FUSE>(a, lg, s, tu); break;
-            default: launch_apply_rk<T, 64, 1, 8, 2, 3, FUSE>(a, lg, s, tu); break;
-            }
+        switch (bcm) {
+        case 0: launch_apply_rk<T, 64, 1, 8, 2, 0, FUSE>(a, lg, s, tu); break;
+        case 1: launch_apply_rk<T, 64, 1, 8, 2, 1, FUSE>(a, lg, s, tu); break;
+        case 2: launch_apply_rk<T, 64, 1, 8, 2, 2, FUSE>(a, lg, s, tu); break;
+        default: launch_apply_rk<T, 64, 1, 8, 2, 3, FUSE>(a, lg, s, tu); break;
         }
     } else if (K == 1 && R == 64 && NW == 8) {
         switch (bcm) {
@@ -1633,10 +1637,10 @@ void apply_impl(tng_operator &op, const tng_vector &src, tng_vector &dst, hipStr
         // penalty: the per-block moments only; every apply workgroup combines them
         const bool pen = op.penalty_active;
         ApplyArgs<T> a = apply_args<T>(op, src, dst, false, add);
-        const ApplyShape sh = apply_shape(m.nr - 1, m.ctx->tuning, false, sizeof(T) == 4);
+        const ApplyShape sh = apply_shape(m.nr - 1, m.ctx->tuning, m.nlat, false, sizeof(T) == 4);
         // partial sums of the levels between radial parts; the allocation-free
         // apply takes the same meshes whether or not its type has parts
-        const int parts = ws ? apply_shape(m.nr - 1, m.ctx->tuning).S : sh.S;
+        const int parts = ws ? apply_shape(m.nr - 1, m.ctx->tuning, m.nlat).S : sh.S;
         if (parts > 1) {
             const size_t bytes = sizeof(T) * 6 * (parts - 1) * (size_t)m.nsd * m.nx * m.nx;
             if (ws) {
@@ -1691,7 +1695,7 @@ bool apply_cheb_impl(tng_operator &op, const tng_vector &x, tng_vector &ax, tng_
         }
         return true;
     }
-    const ApplyShape sh = apply_shape(m.nr - 1, m.ctx->tuning, true, sizeof(T) == 4);
+    const ApplyShape sh = apply_shape(m.nr - 1, m.ctx->tuning, m.nlat, true, sizeof(T) == 4);
     if (!(sh.R == 64 && sh.K <= 2 && sh.NW == 8 && sh.RG <= 2 && sh.S == 1)) return false;
     tng_context &ctx = *m.ctx;
     hipEvent_t *ev = ctx.profiling ? ctx.prof_next_set() : nullptr;

@@ -281,6 +281,24 @@ def test_fp32_pairs_of_cells_match_oracle(L, ls, rs, bcs, gpu_ctx):
         assert rel_err(out.download(), ref) < 1e-5
 
 
+# chunks (the fused step below 2048 columns), parts and pairs of cells form the same products per level
+@pytest.mark.parametrize("L", [3, 4])
+def test_fp32_shapes_at_128_layers_have_the_same_bits(L, gpu_ctx):
+    om = O.Mesh(L, 7)
+    eta, b = np.exp(0.5 * field(om, 1, 39)), field(om, 3, 40)
+    out = []
+    for fuse, split in ((0, 0), (1, 0), (1, 1)):
+        with tng.default_context().tuning(cheb_fuse=fuse, apply_radial_split=split):
+            S = tng.StokesSolver(1, L, 0.55, 1.0, (D, F), tng.StokesParams.defaults(
+                viscous_pc_dtype=tng.F32, viscous_pc_chebyshev_order=3, coarse_solver=1), radial_extra_levels=7 - L)
+            S.set_viscosity(vec(S.domain_velocity, eta))
+            x = tng.VectorQ1Vec(S.domain_velocity)
+            for _ in range(2):
+                S.precondition_velocity(x, vec(S.domain_velocity, b))
+            out.append(x.download())
+    assert all(np.array_equal(out[0], o) for o in out)
+
+
 @pytest.mark.parametrize("bcs", [(D, D), (F, F), (D, F)])
 def test_fp32_pairs_fused_have_the_bits_of_the_separate_kernels(bcs, gpu_ctx):
     om = O.Mesh(4, 7, 0.55, 1.0, 0, 0)
