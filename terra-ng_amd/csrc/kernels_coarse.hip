@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "tng_coarse.hpp"
+#include "tng_wedge.hpp"
 
 namespace tng {
 
@@ -368,7 +369,8 @@ __host__ __device__ __forceinline__ void wedge_around(int q, int &dx, int &dy, i
 }
 
 struct CpcgArgs {
-    const double *lmat;
+    const double *lmat;      // stored wedge matrices, or nullptr: formed from the coefficient
+    const double *k, *radii;
     const int32_t *rep, *copy_begin, *copy_list;
     const uint8_t *slot;
     const double *coords;
@@ -378,31 +380,67 @@ struct CpcgArgs {
     int nu, nx, nr, bc_cmb, bc_surf;
 };
 
-// Sum of the wedge matrices' 3 x 3 blocks into the row's slots; one thread per
-// (node, entry), which owns that entry of every slot of the row.
+// Entry (d1, d2) of the blocks of node i's row of a wedge matrix:
+// k |det J| [ (g_i . g_j) d_{d1,d2} + g_i[d2] g_j[d1] - 2/3 g_i[d1] g_j[d2] ].
+__device__ __forceinline__ void cpcg_row(const double (&g)[6][3], double jkw, int i, int d1, int d2, double (&m)[6])
+{
+    auto pick = [](const double *v, int d) { return d == 0 ? v[0] : (d == 1 ? v[1] : v[2]); };
+    double gi[3] = {g[0][0], g[0][1], g[0][2]};
+#pragma unroll
+    for (int n = 1; n < 6; ++n)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) gi[c] = n == i ? g[n][c] : gi[c];
+    const double gi1 = pick(gi, d1), gi2 = pick(gi, d2);
+#pragma unroll
+    for (int j = 0; j < 6; ++j) {
+        const double gg = gi[0] * g[j][0] + gi[1] * g[j][1] + gi[2] * g[j][2];
+        m[j] = jkw * ((d1 == d2 ? gg : 0.0) + gi2 * pick(g[j], d1) - (2.0 / 3.0) * gi1 * pick(g[j], d2));
+    }
+}
+
+// Sum of the wedge matrices' 3 x 3 blocks into the row's slots: four threads per
+// (node, entry), each with a quarter of the wedges around the node, sum that
+// entry of every slot in LDS.  Without stored matrices the blocks come from the
+// coefficient as they are needed.  Bound by the chain of loads and divisions per
+// wedge.
 __global__ __launch_bounds__(64) void cpcg_assemble_kernel(const CpcgArgs a)
 {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= a.nu * 9) return;
-    const int u = t / 9, e = t - 9 * u, d1 = e / 3, d2 = e - 3 * d1;
+    const int t = (blockIdx.x * blockDim.x + threadIdx.x) >> 2, part = threadIdx.x & 3;
+    const bool live = t < a.nu * 9;
+    const int u = live ? t / 9 : 0, e = t - 9 * u, d1 = e / 3, d2 = e - 3 * d1;
     constexpr int W = CoarsePcg::kWidth;
-    double *row = a.A + ((int64_t)u * 9 + e) * W;
+    __shared__ double rows[64][W + 1];
+    double *row = rows[threadIdx.x];
     for (int s = 0; s < W; ++s) row[s] = 0.0;
     const int nx = a.nx, nr = a.nr, nc = nx - 1, ncr = nr - 1;
-    for (int j = a.copy_begin[u]; j < a.copy_begin[u + 1]; ++j) {
+    for (int j = a.copy_begin[u]; live && j < a.copy_begin[u + 1]; ++j) {
         const int i = a.copy_list[j];
         const int l = i % nr, c = i / nr, Y = c % nx, X = (c / nx) % nx, sd = c / (nx * nx);
-        for (int q = 0; q < 12; ++q) {
+        for (int q = part; q < 12; q += 4) {
             int dx, dy, w, dr, corner;
             wedge_around(q, dx, dy, w, dr, corner);
             const int xc = X + dx, yc = Y + dy, rc = l + dr;
             if (xc < 0 || xc >= nc || yc < 0 || yc >= nc || rc < 0 || rc >= ncr) continue;
-            const double *m = a.lmat + (((((int64_t)sd * nc + xc) * nc + yc) * ncr + rc) * 2 + w) * 324 +
-                              (corner + (dr == 0 ? 0 : 3) + 6 * d1) * 18 + 6 * d2;
+            const int node = corner + (dr == 0 ? 0 : 3);
+            double m[6];
+            if (a.lmat) {
+                const double *l = a.lmat + (((((int64_t)sd * nc + xc) * nc + yc) * ncr + rc) * 2 + w) * 324 +
+                                  (node + 6 * d1) * 18 + 6 * d2;
+                for (int k = 0; k < 6; ++k) m[k] = l[k];
+            } else {
+                double g[6][3], jkw;
+                wedge_gradients(a.coords, a.radii, a.k, nx, nr, sd, xc, yc, rc, w, g, &jkw);
+                cpcg_row(g, jkw, node, d1, d2, m);
+            }
             const uint8_t *sl = a.slot + (int64_t)i * CoarsePcg::kMaxSlots + 6 * q;
             for (int k = 0; k < 6; ++k) row[sl[k]] += m[k];
         }
     }
+    __syncthreads();
+    if (!live) return;
+    const double(*r)[W + 1] = rows + (threadIdx.x & ~3);
+    double *out = a.A + ((int64_t)u * 9 + e) * W;
+    for (int s = part; s < W; s += 4) out[s] = (r[0][s] + r[1][s]) + (r[2][s] + r[3][s]);
 }
 
 // kind of a node: 0 interior or Neumann, else its boundary condition; n its unit normal
@@ -665,10 +703,12 @@ void CoarsePcg::build(tng_operator &A, hipStream_t s)
 {
     const tng_domain &m = *A.mesh;
     if (!d_uid.p) numbering(m);
-    if (!A.stored) epsdivdiv_local_matrices(A, d_local, s);
-    TNG_REQUIRE(!A.stored || A.lmat_dtype == TNG_F64, "coarse PCG: FP64 matrices required");
+    TNG_REQUIRE(A.stored ? A.lmat_dtype == TNG_F64 : A.k && A.k->dtype == TNG_F64,
+                "coarse PCG: FP64 matrices or an FP64 coefficient required");
     CpcgArgs a{};
-    a.lmat = A.stored ? A.d_lmat.as<double>() : d_local.as<double>();
+    a.lmat = A.stored ? A.d_lmat.as<double>() : nullptr;
+    a.k = A.k ? (const double *)A.k->comp(0) : nullptr;
+    a.radii = m.d_radii.as<double>();
     a.rep = d_rep.as<int32_t>();
     a.copy_begin = d_copy_begin.as<int32_t>();
     a.copy_list = d_copy_list.as<int32_t>();
@@ -679,7 +719,7 @@ void CoarsePcg::build(tng_operator &A, hipStream_t s)
     a.sd_surf = m.d_sd_surf.as<uint8_t>();
     a.A = d_A.as<double>();
     a.nu = nu; a.nx = m.nx; a.nr = m.nr; a.bc_cmb = A.bc_cmb; a.bc_surf = A.bc_surf;
-    hipLaunchKernelGGL(cpcg_assemble_kernel, dim3((nu * 9 + 63) / 64), dim3(64), 0, s, a);
+    hipLaunchKernelGGL(cpcg_assemble_kernel, dim3((nu * 36 + 63) / 64), dim3(64), 0, s, a);
     hipLaunchKernelGGL(cpcg_boundary_kernel, dim3((nu * kWidth + 63) / 64), dim3(64), 0, s, a);
     TNG_HIP_CHECK(hipGetLastError());
     ready = true;

@@ -34,7 +34,7 @@ struct CoarsePcg {
     int nu = 0;
     int64_t ncopies = 0;
     bool ready = false;
-    DevBuf d_uid, d_rep, d_slot, d_col, d_copy_begin, d_copy_list, d_A, d_vec, d_state, d_local;
+    DevBuf d_uid, d_rep, d_slot, d_col, d_copy_begin, d_copy_list, d_A, d_vec, d_state;
     // the operator is a plain one (no rotation penalty) on a mesh of this size
     static bool accepts(const tng_operator &A);
     void numbering(const tng_domain &m);

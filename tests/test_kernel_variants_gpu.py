@@ -114,6 +114,17 @@ def test_assembled_coarse_pcg_solves_the_coarse_system(bcs, gca, sdr, dtype, gpu
     assert rel_err(out[1], out[0]) < (1e-8 if dtype == tng.F64 else 1e-6)
 
 
+# a new viscosity assembles that operator; with the rotation penalty, whose coarse PCG is not assembled, it does not
+def test_assembled_coarse_operator_costs_little_per_viscosity(gpu_ctx):
+    times = []
+    for bcs in ((D, F), (F, F)):
+        S = tng.StokesSolver(2, 3, 0.55, 1.0, bcs, tng.StokesParams.defaults(krylov_restart=2))
+        eta = tng.VectorQ1Scalar(S.domain_velocity)
+        eta.fill(1.0)
+        times.append(microseconds(S.domain_velocity, lambda: S.set_viscosity(eta)))
+    assert times[0] < 2 * times[1]
+
+
 # launches after the end of a coarse solve change nothing, wherever in the host's look at the end (every 25) it falls:
 # ended by the tolerance within the first 25 iterations, and by a zero right-hand side, for which p.(A p) is zero
 @pytest.mark.parametrize("dtype", [tng.F64, tng.F32])
