@@ -1645,10 +1645,10 @@ void apply_impl(tng_operator &op, const tng_vector &src, tng_vector &dst, hipStr
             const size_t bytes = sizeof(T) * 6 * (parts - 1) * (size_t)m.nsd * m.nx * m.nx;
             if (ws) {
                 TNG_REQUIRE(bytes <= kNoAllocScratchBytes - kNoAllocPenDoubles * sizeof(double),
-                            "allocation-free apply: the partial sums between radial parts need " +
-                                std::to_string(bytes) + " bytes, more than the " +
+                            "allocation-free apply: meshes whose partial sums between radial parts (here " +
+                                std::to_string(bytes) + " bytes) exceed the " +
                                 std::to_string(kNoAllocScratchBytes - kNoAllocPenDoubles * sizeof(double)) +
-                                " bytes of scratch");
+                                " bytes of scratch are not taken, whether or not this precision sweeps in parts");
                 a.iface = reinterpret_cast<T *>(ws + kNoAllocPenDoubles);
             } else {
                 if (op.d_iface.bytes < bytes) op.d_iface.alloc(bytes);
