@@ -85,9 +85,11 @@ template <typename T> struct ApplyArgs {
     T *cd0, *cd1, *cd2, *cx0, *cx1, *cx2;
     T caz, cad;
     int cread_d;
-    // the radii in FP64 for FP32 applies: a layer's thickness is the difference
-    // of two radii, of which FP32 values keep few digits (128 layers: 1e-5 relative)
-    const double *radii64;
+    // FP32 applies: q and cv of each layer, formed in FP64 with the mesh.  A
+    // layer's thickness is the difference of two radii, of which FP32 values keep few
+    // digits (128 layers: 1e-5 relative), and three FP64 divisions per lane are 0.3 us
+    // of a small mesh's 20
+    const T *layer;
 };
 
 template <typename T> __device__ __forceinline__ void normal_of(const T *c, T n[3])
@@ -508,18 +510,17 @@ __global__ __launch_bounds__(NW * 64) void epsdivdiv_apply_kernel(const ApplyArg
     #pragma unroll
         for (int p = 0; p < K; ++p) {
             const int l = lvl0 + p;
-            double r0, r1;
             if constexpr (sizeof(T) == 8) {
-                r0 = a.radii[(int64_t)sd * nr + l];
-                r1 = a.radii[(int64_t)sd * nr + l + 1];
+                const T r0 = a.radii[(int64_t)sd * nr + l], r1 = a.radii[(int64_t)sd * nr + l + 1];
+                const T rmid = T(0.5) * (r0 + r1), h = T(0.5) * (r1 - r0);
+                const T hs = T(0.5) / rmid, tt = T(1) / (T(6) * h);
+                qq[p] = tt / hs;
+                cv[p] = lane_has ? hs * hs * rmid * rmid * h * T(1.0 / 6.0) : T(0);
             } else {
-                r0 = a.radii64[(int64_t)sd * nr + l];
-                r1 = a.radii64[(int64_t)sd * nr + l + 1];
+                const T *y = a.layer + 2 * ((int64_t)sd * a.ncells + l);
+                qq[p] = y[0];
+                cv[p] = lane_has ? y[1] : T(0);
             }
-            const double rmid = 0.5 * (r0 + r1), h = 0.5 * (r1 - r0);
-            const double hs = 0.5 / rmid, tt = 1.0 / (6.0 * h);
-            qq[p] = (T)(tt / hs);
-            cv[p] = lane_has ? (T)(hs * hs * rmid * rmid * h * (1.0 / 6.0)) : T(0);
         }
 
         auto colbase = [&](int Xq, int Yq) -> int64_t {
@@ -1589,7 +1590,7 @@ ApplyArgs<T> apply_args(const tng_operator &op, const tng_vector &src, tng_vecto
     a.dst0 = (T *)dst.comp(0); a.dst1 = (T *)dst.comp(1); a.dst2 = (T *)dst.comp(2);
     a.k = (const T *)op.k->comp(0);
     a.radii = mp.radii; a.latgeom = mp.latgeom; a.coords = mp.coords;
-    a.radii64 = m.d_radii.as<double>();
+    if constexpr (sizeof(T) == 4) a.layer = m.d_layer_f.as<float>();
     a.btab = op.d_btab.as<T>();
     a.pen = pen ? op.d_penalty_b.as<double>() : nullptr;
     a.sd_cmb = m.d_sd_cmb.as<uint8_t>(); a.sd_surf = m.d_sd_surf.as<uint8_t>();

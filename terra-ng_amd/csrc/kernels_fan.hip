@@ -28,7 +28,7 @@ template <typename T> struct FanArgs {
     const T *src[3];
     T *dst[3];  // A x; with the sub-step: x + d
     const T *k, *latgeom, *coords, *btab;
-    const double *radii;  // FP64 in either precision: FP32 radii keep few digits of a layer's thickness
+    const double *radii;  // FP64
     const uint8_t *sd_cmb, *sd_surf;
     const int32_t *task_col, *task_grp;  // (block, slot): lateral column or -1; first | count << 8 of its copies
     int nx, bc_cmb, bc_surf, add, sum;
@@ -38,6 +38,7 @@ template <typename T> struct FanArgs {
     T *d[3];
     T az, ad;
     int read_d;
+    const T *layer;  // FP32: q and cv of each layer, formed in FP64 with the mesh
 };
 
 enum { FAN_APPLY = 0, FAN_CHEB = 1 };
@@ -206,10 +207,17 @@ __global__ __launch_bounds__(kFanBlock<R>) void fan_kernel(const FanArgs<T> a)
     fan_load(a, col, nr, rl, rp);
 #pragma unroll
     for (int n = 0; n < 4; ++n) fan_load(a, neighbour(n), nr, rl, rn[n]);
-    const double r0 = a.radii[sd * nr + rl], r1 = a.radii[sd * nr + rl + 1];
-    const double rmid = 0.5 * (r0 + r1), h = 0.5 * (r1 - r0), hs = 0.5 / rmid;
-    const T q = (T)((1.0 / (6.0 * h)) / hs);
-    const T cv = (T)(hs * hs * rmid * rmid * h * (1.0 / 6.0));
+    T q, cv;
+    if constexpr (sizeof(T) == 8) {
+        const double r0 = a.radii[sd * nr + rl], r1 = a.radii[sd * nr + rl + 1];
+        const double rmid = 0.5 * (r0 + r1), h = 0.5 * (r1 - r0), hs = 0.5 / rmid;
+        q = (1.0 / (6.0 * h)) / hs;
+        cv = hs * hs * rmid * rmid * h * (1.0 / 6.0);
+    } else {
+        const T *y = a.layer + 2 * (sd * R + rl);
+        q = y[0];
+        cv = y[1];
+    }
     T L[3] = {T(0), T(0), T(0)}, C[3] = {T(0), T(0), T(0)};
     const FanCol<T> P = fan_column<T, BCM>(a, col, rp, bc);
     FanCol<T> prev = fan_column<T, BCM>(a, neighbour(0), rn[0], bc);
@@ -327,6 +335,7 @@ template <typename T> FanArgs<T> fan_args(const tng_operator &op, const tng_vect
     constexpr bool f64 = sizeof(T) == 8;
     a.k = (const T *)op.k->comp(0);
     a.radii = m.d_radii.as<double>();
+    if constexpr (!f64) a.layer = m.d_layer_f.as<float>();
     a.latgeom = (const T *)(f64 ? m.d_latgeom.p : m.d_latgeom_f.p);
     a.coords = (const T *)(f64 ? m.d_coords.p : m.d_coords_f.p);
     a.btab = op.d_btab.as<T>();

@@ -341,6 +341,14 @@ void mesh_upload(tng_domain &m)
     std::vector<float> cf(m.coords.begin(), m.coords.end()), rf(m.radii.begin(), m.radii.end());
     up(m.d_coords_f, cf.data(), cf.size() * sizeof(float));
     up(m.d_radii_f, rf.data(), rf.size() * sizeof(float));
+    std::vector<float> lf;
+    for (int sd = 0; sd < m.nsd; ++sd)
+        for (int l = 0; l + 1 < m.nr; ++l) {
+            const double r0 = m.radii[(size_t)sd * m.nr + l], r1 = m.radii[(size_t)sd * m.nr + l + 1];
+            lf.push_back((float)((r0 + r1) / (3.0 * (r1 - r0))));
+            lf.push_back((float)((r1 - r0) / 48.0));
+        }
+    up(m.d_layer_f, lf.data(), lf.size() * sizeof(float));
 
     // lateral wedge geometry (sd, xc, yc, w, 10)
     const int nc = nx - 1;

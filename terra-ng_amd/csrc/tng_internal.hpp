@@ -159,6 +159,7 @@ struct tng_domain {
     // device copies
     tng::DevBuf d_coords, d_radii, d_omask, d_bmask, d_sd_cmb, d_sd_surf;
     tng::DevBuf d_coords_f, d_radii_f;
+    tng::DevBuf d_layer_f;  // FP32 applies: (sd, layer, 2) = (rmid / (3h), h / 24), h half the thickness
     // lateral wedge geometry: (sd, xc, yc, wedge, 10) = (M0, M1, M2, |det L|),
     // M = columns of L^{-T}, L = [p1-p0, p2-p0, (p0+p1+p2)/3]
     tng::DevBuf d_latgeom, d_latgeom_f;
