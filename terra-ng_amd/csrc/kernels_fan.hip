@@ -3,9 +3,9 @@
 // included: one launch for what the sweeping apply, the halo sum and the
 // vector update do in three (the discretisation and its references are those
 // of kernels_epsdivdiv.hip).  Sub-step of the smoother, FP32 no-slip: level 3
-// 20.8 -> 6.6 us, level 4 22 -> 7.4 us, level 5 31.7 -> 20.9 us; FP64: level 3
-// 19 -> 8.2 us, level 4 20 -> 12 us.  Apply with halo sum alone, level 4 FP64:
-// 15.9 -> 9 us.
+// 20.8 -> 6.6 us, level 4 22 -> 7.3 us, level 5 31.7 -> 20.4 us; FP64: level 3
+// 19 -> 8.6 us, level 4 20 -> 11.5 us.  Apply with halo sum alone, level 4 FP64:
+// 13.5 -> 7.6 us.
 //
 // What bounds these sizes is not arithmetic or bandwidth but launches and the
 // chain inside one: a sweep over a row of cells is a serial loop of loads,
@@ -155,8 +155,9 @@ __device__ __forceinline__ void fan_triangle(const FanCol<T> &P, const FanCol<T>
 
 // Two groups of R lanes per node copy, three triangles each: half the chain of
 // a group that takes all six (levels 3 and 4: 8.6 and 8.4 us per FP32 sub-step
-// with one group, 6.6 and 7.4 with two; level 5 18.5 and 20.9), and registers
-// for more waves per SIMD.
+// with one group, 6.6 and 7.4 with two).  At level 5, where the chip is full,
+// one group was the faster by a tenth (18.5 against 20.9 us); 32 layers take two
+// like the rest, for one layout of table, block and epilogue.
 template <int R> constexpr int kFanBlock = R == 32 ? 512 : 256;
 template <int R> constexpr int kFanCap = kFanBlock<R> / (2 * R);  // node copies per block, at least 8
 
