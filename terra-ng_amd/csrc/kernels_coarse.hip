@@ -345,7 +345,8 @@ void CoarseDirect::solve(tng_vector &e0, const tng_vector &r0, hipStream_t s)
 // against 3.3 MB of wedge matrices, most of which five blocks of gathering
 // threads read per apply), and each of an iteration's two reductions ends in
 // the next kernel, where every block sums the partials itself.  Level 2 (810
-// nodes), Galerkin operator: 8.8 us per iteration (5.2 + 3.6), 71 us with the
+// nodes), Galerkin operator: 8.8 us of kernel time per iteration (5.2 + 3.6; 9.0
+// with the gaps, 0.45 ms for 50), 71 us with the
 // stored-matrix apply, halo sum and five vector kernels.  Used up to 8192
 // nodes (lateral level 3), where the matrix kernel's 10 MB still come from
 // cache; above, and with the rotation penalty (a rank-3 term over all nodes),

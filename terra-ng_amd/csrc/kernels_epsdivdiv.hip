@@ -1378,8 +1378,9 @@ ApplyShape apply_shape(int ncells, const tng_tuning &tu, int64_t columns, bool f
         // with two chunks, 810 columns 20.6 against 15.4, 2890 columns 21.2 against
         // 22.8.  An apply spares a launch: 250 columns 18.2 us against 18.0 in two
         // parts (with the rotation penalty 26.6 against 27.4), 810 columns 18.6
-        // against 18.7, 2890 columns 19.0 against 19.3.  FP64 takes 64 cells per lane set: two cells of it exceed the 256
-        // registers that two waves per SIMD leave.
+        // against 18.7, 2890 columns 19.0 against 19.3.  FP64 takes 64 cells per
+        // lane set: two cells of it exceed the 256 registers that two waves per SIMD
+        // leave.
         sh.K = 2;
         return sh;
     }
