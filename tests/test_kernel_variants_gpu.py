@@ -254,7 +254,7 @@ def test_small_divergence_takes_no_longer_in_fp64(gpu_ctx):
         u.fill(1.0)
         op = tng.DivergenceKerngen(fine, coarse, (D, F))
         times.append(microseconds(fine, lambda: op.apply(u, out)))
-    assert times[0] < 1.05 * times[1]
+    assert times[0] < 1.08 * times[1]  # 0.94; 1.12 with one pass
 
 
 # spare vectors of the fused sub-step only where a level takes it: none with the rotation penalty below 64 layers
